@@ -1,0 +1,46 @@
+"""Batched prefill per weight type and token count vs the CPU oracle (MI355X).
+
+Tolerances: activations and weights meet as 22-bit f16 pairs and f32 sums, so
+a product is off by about 1e-6 of its magnitude; logits of these two-layer
+models (order 1) may be off by 2e-4 (the quantized LM head's 15-bit activation
+digits among it) and K/V rows (order 1) by 2e-5.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from hf_checkpoint import write_checkpoint
+
+pytestmark = pytest.mark.gpu
+
+
+def check(llrs, oracle, model, tmp_path, vocab, layers, n, seed):
+    model.export_gguf(tmp_path / "m.gguf")
+    om = oracle.load(tmp_path / "m.gguf")
+    om.new_state(n + 4)
+    kv = llrs.KVCache(model, n + 4)
+    prompt = np.random.default_rng(seed).integers(0, vocab, n).astype(np.uint32)
+    model.prefill(prompt, 0, kv)
+    om.prefill(prompt, 0)
+    err = float(np.abs(kv.logits() - om.logits()).max())
+    print(f"[types] n={n} logits max-abs err {err:.3e}", flush=True)
+    assert err <= 2e-4 * max(1.0, float(np.abs(om.logits()).max()))
+    for layer in range(layers):
+        for which in ("k", "v"):
+            a, b = kv.layer(layer, which, n), om.kv(layer, which, n)
+            assert float(np.abs(a - b).max()) <= 2e-5 * max(1.0, float(np.abs(b).max())), (layer, which)
+
+
+@pytest.mark.parametrize("n", [2, 65, 257], ids=["2", "65", "257"])
+@pytest.mark.parametrize("dtype", ["BF16", "F16", "F32"])
+def test_prefill_float_weights(llrs, backend, oracle, tmp_path, dtype, n):
+    """Unquantized checkpoints: FFN matrices of 2,080 rows (sixteen 128-row
+    tiles and a remainder), two tokens, one past a 64-token tile, one past
+    two 128-token tiles."""
+    cfg = llrs.SynthConfig(hidden_size=256, intermediate_size=2080, num_attention_heads=4, num_key_value_heads=2,
+                           num_hidden_layers=2, vocab_size=1000, max_position_embeddings=512, seed=51,
+                           tie_word_embeddings=False)
+    write_checkpoint(llrs, cfg, tmp_path / "ck", dtype)
+    model = llrs.ModelLoader.load(tmp_path / "ck", backend)
+    check(llrs, oracle, model, tmp_path, cfg.vocab_size, cfg.num_hidden_layers, n, 51 + n)
