@@ -1415,11 +1415,12 @@ static int sample_with(llrs_kv *kv, const llrs_sampling *opts, const uint32_t *r
   llrs_model *m = kv->m;
   hipStream_t s = m->b->stream;
   const int V = (int)m->cfg.vocab_size;
-  if (n_recent) LLRS_HIP(hipMemcpyAsync(w.recent, recent, n_recent * 4, hipMemcpyHostToDevice, s));
   const SampleParams p{opts->temperature, (int)std::min<uint32_t>(opts->top_k, (uint32_t)V), opts->top_p,
                        opts->repetition_penalty};
-  LLRS_TRY(launch_sample(kv->logits, V, p, (int)n_recent, uniform, w, s));
-  LLRS_HIP(hipMemcpyAsync(kv->pinned, w.token, 4, hipMemcpyDeviceToHost, s));
+  // The kernel writes the token into the cache's pinned host words itself.
+  uint32_t *out = nullptr;
+  LLRS_HIP(hipHostGetDevicePointer((void **)&out, kv->pinned, 0));
+  LLRS_TRY(launch_sample(kv->logits, V, p, recent, (int)n_recent, uniform, w, out, s));
   LLRS_HIP(hipStreamSynchronize(s));
   *out_token = kv->pinned[0];
   return LLRS_OK;
@@ -1727,12 +1728,11 @@ int llrs_sample(llrs_kv *kv, const llrs_sampling *opts, const uint32_t *recent, 
   if (!w.n) {
     auto A = [&](void **p, size_t bytes) { return dev_alloc(kv->allocs, p, bytes); };
     w.tmp_bytes = sample_sort_bytes(V);
-    LLRS_TRY(A((void **)&w.keys, (size_t)V * 4));
+    LLRS_TRY(A((void **)&w.keys, ((size_t)V + 3) / 4 * 16));  // read four keys at a time
     LLRS_TRY(A((void **)&w.keys_sorted, (size_t)V * 4));
     LLRS_TRY(A((void **)&w.idx, (size_t)V * 4));
     LLRS_TRY(A((void **)&w.idx_sorted, (size_t)V * 4));
     LLRS_TRY(A((void **)&w.recent, kMaxRecent * 4));
-    LLRS_TRY(A((void **)&w.token, 64));
     LLRS_TRY(A(&w.tmp, w.tmp_bytes ? w.tmp_bytes : 1));
     w.max_recent = (int)kMaxRecent;
     w.n = V;

@@ -17,11 +17,11 @@ struct SampleParams {
 };
 
 // Device scratch for a vocabulary of n tokens: sort keys and indices (in and
-// out), the radix sort's temporary storage, the repeat window, the result.
+// out), the radix sort's temporary storage, the repeat window.
 struct SampleScratch {
   int n = 0, max_recent = 0;
   uint32_t *keys = nullptr, *keys_sorted = nullptr, *idx = nullptr, *idx_sorted = nullptr;
-  uint32_t *recent = nullptr, *token = nullptr;
+  uint32_t *recent = nullptr;
   void *tmp = nullptr;
   size_t tmp_bytes = 0;
 };
@@ -41,9 +41,13 @@ constexpr size_t kNoAllocSortBytes = 4u << 20;
 // storage than kNoAllocSortBytes.  Every call on one device shares the array.
 int sample_noalloc_scratch(SampleScratch &w);
 
-// Samples from logits[0, n) into *w.token (device), using the uniform draw u
-// in [0, 1); recent[0, n_recent) is already on the device (w.recent).
-int launch_sample(const float *logits, int n, const SampleParams &p, int n_recent, float u,
-                  SampleScratch &w, hipStream_t s);
+// Windows of up to this many tokens travel as a kernel argument.
+constexpr int kArgRecent = 256;
+
+// Samples from logits[0, n) into *out (memory the device can write, for
+// instance mapped host memory), using the uniform draw u in
+// [0, 1); recent[0, n_recent) is the repeat window in host memory.
+int launch_sample(const float *logits, int n, const SampleParams &p, const uint32_t *recent, int n_recent, float u,
+                  SampleScratch &w, uint32_t *out, hipStream_t s);
 
 }  // namespace llrs
