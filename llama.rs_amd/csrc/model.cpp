@@ -1229,12 +1229,12 @@ static int prefill_gemm(llrs_kv *kv, const llrs_tensor *w, const f16 *a, const f
 }
 
 // Whether gate and up run as one dual product with SwiGLU in its epilogue:
-// both Q4_K on their codes, the FFN width a multiple of 64 (unless
-// LLRS_PREFILL_DUAL=0, read per call, for comparisons).
-static bool use_dual_gate_up(const DevLayer &L, int F) {
+// both of one type whose products fuse, the FFN width a multiple of 64
+// (unless LLRS_PREFILL_DUAL=0, read per call, for comparisons).
+static bool use_dual_gate_up(const DevLayer &L, int F, int T) {
   const char *e = getenv("LLRS_PREFILL_DUAL");
-  return !(e && strcmp(e, "0") == 0) && L.gate->type == LLRS_Q4_K && L.up->type == LLRS_Q4_K &&
-         L.gate->row_bytes == L.up->row_bytes && F % 64 == 0 && prefill_codes_enabled();
+  return !(e && strcmp(e, "0") == 0) && L.gate->type == L.up->type && L.gate->row_bytes == L.up->row_bytes &&
+         F % 64 == 0 && prefill_fuses(L.gate->type, L.gate->row_bytes, 2 * F, T);
 }
 
 // silu(gate) * up as f16 pairs into h/hl [T][F] (and, for a Q4_K ffn_down,
@@ -1247,12 +1247,14 @@ static int prefill_gate_up_dual(llrs_kv *kv, const DevLayer &L, int H, int F, in
   g.a = kv->pf_h;
   g.a_lo = kv->pf_hl;
   g.lda = H;
-  g.xs = kv->pf_xs;
-  g.xs_lo = kv->pf_xsl;
-  g.ldxs = kv->pf_ldxs;
+  if (L.gate->type == LLRS_Q4_K) {
+    g.xs = kv->pf_xs;
+    g.xs_lo = kv->pf_xsl;
+    g.ldxs = kv->pf_ldxs;
+  }
   g.w = L.gate->dev;
   g.w2 = L.up->dev;
-  g.type = LLRS_Q4_K;
+  g.type = L.gate->type;
   g.row_bytes = (long)L.gate->row_bytes;
   g.dual_rows = F;
   g.n = 2 * F;
@@ -1269,30 +1271,32 @@ static int prefill_gate_up_dual(llrs_kv *kv, const DevLayer &L, int H, int F, in
   return launch_prefill_gemm(g, s);
 }
 
-// Q, K (and V when it is Q4_K too) of one input as one segmented Q4_K product
-// over pf_h (one launch and one split-K reduction instead of two or three):
-// when they all run on their codes and every boundary is a multiple of 128
+// Q, K (and V when it has their type too) of one input as one segmented
+// product over pf_h (one launch and one split-K reduction instead of two or
+// three): when the type's products fuse and every boundary is a multiple of 128
 // rows (unless LLRS_PREFILL_QKV=0, read per call, for comparisons).  Returns
 // whether V was included; sets *done when the product ran.
 static int prefill_qkv_segmented(llrs_kv *kv, const DevLayer &L, int H, int KV, int T, bool &done,
                                  bool &with_v, hipStream_t s) {
   done = with_v = false;
   const char *e = getenv("LLRS_PREFILL_QKV");
-  if ((e && strcmp(e, "0") == 0) || !prefill_codes_enabled() || L.q->type != LLRS_Q4_K ||
-      L.k->type != LLRS_Q4_K || L.k->row_bytes != L.q->row_bytes || H % 128)
+  if ((e && strcmp(e, "0") == 0) || !prefill_fuses(L.q->type, L.q->row_bytes, H + 2 * KV, T) || L.k->type != L.q->type ||
+      L.k->row_bytes != L.q->row_bytes || H % 128)
     return LLRS_OK;
-  with_v = L.v->type == LLRS_Q4_K && L.v->row_bytes == L.q->row_bytes && KV % 128 == 0;
+  with_v = L.v->type == L.q->type && L.v->row_bytes == L.q->row_bytes && KV % 128 == 0;
   PrefillGemmArgs g{};
   g.part = kv->pf_part;
   g.part_cap = kv->pf_part_cap;
   g.a = kv->pf_h;
   g.a_lo = kv->pf_hl;
   g.lda = H;
-  g.xs = kv->pf_xs;
-  g.xs_lo = kv->pf_xsl;
-  g.ldxs = kv->pf_ldxs;
+  if (L.q->type == LLRS_Q4_K) {
+    g.xs = kv->pf_xs;
+    g.xs_lo = kv->pf_xsl;
+    g.ldxs = kv->pf_ldxs;
+  }
   g.w = L.q->dev;
-  g.type = LLRS_Q4_K;
+  g.type = L.q->type;
   g.row_bytes = (long)L.q->row_bytes;
   g.k = H;
   g.t = T;
@@ -1343,7 +1347,7 @@ static int prefill_batched(llrs_model *m, llrs_kv *kv, size_t start, size_t n) {
       LLRS_TRY(launch_rmsnorm_rows_f16(kv->pf_x, L.attn_norm, kv->pf_h, kv->pf_hl, T, H, eps, s,
                                        xs ? kv->pf_xs : nullptr, kv->pf_xsl, kv->pf_ldxs));
       bool qk_done = false, with_v = false;
-      if (xs) LLRS_TRY(prefill_qkv_segmented(kv, L, H, KV, T, qk_done, with_v, s));
+      LLRS_TRY(prefill_qkv_segmented(kv, L, H, KV, T, qk_done, with_v, s));
       if (!qk_done) {
         LLRS_TRY(prefill_gemm(kv, L.q, kv->pf_h, kv->pf_hl, H, kv->pf_q, H, L.bq, T, false, xs, s));
         LLRS_TRY(prefill_gemm(kv, L.k, kv->pf_h, kv->pf_hl, H, kv->pf_k, KV, L.bk, T, false, xs, s));
@@ -1359,7 +1363,7 @@ static int prefill_batched(llrs_model *m, llrs_kv *kv, size_t start, size_t n) {
       xs = needs_xsum({L.gate, L.up});
       LLRS_TRY(launch_rmsnorm_rows_f16(kv->pf_x, L.ffn_norm, kv->pf_h, kv->pf_hl, T, H, eps, s,
                                        xs ? kv->pf_xs : nullptr, kv->pf_xsl, kv->pf_ldxs));
-      if (xs && use_dual_gate_up(L, F)) {
+      if (use_dual_gate_up(L, F, T)) {
         // SwiGLU in the product's epilogue: its f16 pairs go to the gate/up
         // scratch (pf_h is this product's input), the sums to pf_xs2.
         f16 *h = reinterpret_cast<f16 *>(kv->pf_g), *hl = reinterpret_cast<f16 *>(kv->pf_u);

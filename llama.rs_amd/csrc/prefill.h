@@ -35,9 +35,9 @@ struct PrefillGemmArgs {
   // runs on the Q4_K codes as exact integers (prefill_codes_enabled()).
   const f16 *xs, *xs_lo;
   int ldxs;
-  // Dual product (gate and up, Q4_K on its codes): w are the gate rows, w2 the
-  // up rows (same k, type and row bytes), n = 2 * dual_rows virtual rows
-  // (each 128-row tile holds 64 gate rows and the same 64 up rows), and the
+  // Dual product (gate and up, a type prefill_fuses): w are the gate
+  // rows, w2 the up rows (same k, type and row bytes), n = 2 * dual_rows virtual
+  // rows (in the split-K partials 64 gate rows, then the same 64 up rows), and the
   // output is silu(gate) * up as f16 pairs h/hl [t][ldh] instead of c; with
   // xso set, also its 32-column sums (for a Q4_K ffn_down).
   const uint8_t *w2;
@@ -46,7 +46,7 @@ struct PrefillGemmArgs {
   int ldh;
   f16 *xso, *xso_lo;
   int ldxso;
-  // Segmented product (Q4_K on its codes, e.g. q, k and v of one input): rows
+  // Segmented product (a type prefill_fuses, e.g. q, k and v of one input): rows
   // [seg_base[i], seg_base[i + 1]) of the n come from seg_w[i] and go to
   // seg_c[i] (row stride seg_ldc[i], bias seg_bias[i] or null); every
   // boundary but the last a multiple of 128.  nseg = 0: w, c, ldc and bias.
@@ -66,6 +66,20 @@ int launch_prefill_gemm(const PrefillGemmArgs &g, hipStream_t s);
 // LLRS_PREFILL_CODES=f32 or the four-wave GEMM, LLRS_PREFILL_GEMM=4, select
 // the f32-weight product).  Read at every call.
 bool prefill_codes_enabled();
+// The register-decoded products (prefill_reg.hip): the types they have, a row
+// wave's weight rows, a workgroup's most row waves (a group) and tokens, and
+// the launch of g's tiles (g.ksplit K ranges; the partials' reduction is the
+// caller's).
+bool prefill_reg_supports(uint32_t type);
+int prefill_reg_row_tile(bool dual);
+int prefill_reg_max_row_waves();
+int prefill_reg_token_tile(uint32_t type, int t);
+int prefill_reg_big_row_tile(uint32_t type, bool dual);
+void launch_prefill_reg(const PrefillGemmArgs &g, int row_waves, hipStream_t s);  // 0: the many-token kernel
+// Whether a product of `rows` rows (row_bytes each) of this type over t tokens runs
+// register-decoded and so may be dual or segmented (LLRS_PREFILL_CODES=f32 or
+// LLRS_PREFILL_GEMM=4 select the LDS-staged product for all).  Read at every call.
+bool prefill_fuses(uint32_t type, size_t row_bytes, int rows, int t);
 // xs + xs_lo [t][s] = sum_{j<32} (a + a_lo)[t][32 s + j] as f16 pairs, s < k/32, t < T.
 int launch_xsum_f16(const f16 *a, const f16 *a_lo, int lda, int k, int T, f16 *xs, f16 *xs_lo, int ldxs,
                     hipStream_t s);

@@ -18,12 +18,12 @@
 // Precision: f32 operands are carried as f16 pairs, v = hi + lo with hi =
 // f16(v) and lo = f16(v - hi) (22 significant bits), and each product is
 // hi*hi + hi*lo + lo*hi (the lo*lo term is below f32 rounding of the sum), so
-// the GEMM is close to an f32 GEMM rather than an f16 one.  Q4_K weights take
-// prefill_gemm_k4_kernel instead: their integer codes are exact f16 values,
-// so one weight plane and two MFMAs per product suffice.
+// the GEMM is close to an f32 GEMM rather than an f16 one.  Most products of
+// the types in prefill_reg.hip take its kernels instead.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstdlib>
 #include <cstring>
 
@@ -343,67 +343,6 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(PrefillGemmArgs g) {
   store_tile<MI, 4>(g, acc, n0 + wn * 64, t0 + wm * (BM / 2), lane);
 }
 
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
-// One staging thread's 32 Q6_K weights of a row (columns col .. col + 31, within
-// one 32-column quarter of a 128-column half) on their integer codes.  A Q6_K
-// weight is d * sc * (q - 32) (value_at, src/quant.rs:349-456): q a 6-bit
-// code, sc an int8 per 16 columns, d per 256-column block.  sc * (q - 32) is
-// an integer of magnitude at most 4,096: hi = its f16 rounding and lo = the
-// remainder (-1, 0 or 1, exact), from packed f16 arithmetic on 1024 + q (the
-// bit pattern 0x6400 | q): q - 32 is exact, hi one product, lo one fma.  d is
-// applied to the accumulators per 256-column block (`first`: this thread
-// keeps the row's unit u and publishes the block's rescale d_prev / d and the
-// unit; a block with d = 0 is staged as zeros and keeps the unit), as in
-// prefill_gemm_k4_kernel.  The three MFMAs per product stay (lo*x_hi is needed
-// where |sc * (q - 32)| > 2,048); the staging drops from ~14 VALU operations
-// per weight to ~3 per two.
-__device__ __forceinline__ void stage_q6k_codes(const Deq<LLRS_Q6_K>::Raw &r, int col, bool w_ok, bool first,
-                                                float &u, float *ratio, float *unit, f16 *ws, f16 *wl) {
-#pragma clang fp contract(off)
-  const float d = f16_bits_to_f32(r.d);
-  const bool live = d != 0.f;  // NaN d is live and makes the row NaN, as in f32
-  if (first) {
-    *ratio = live ? u / d : 1.f;
-    if (live) u = d;
-    *unit = u;
-  }
-  const int quarter = (col >> 5) & 3;
-  const bool use = w_ok && live;
-  const f16 s0 = (f16)(float)(use ? (int)(int8_t)(r.s2 & 0xff) : 0);
-  const f16 s1 = (f16)(float)(use ? (int)(int8_t)(r.s2 >> 8) : 0);
-  const half2v off = {(f16)-1056.f, (f16)-1056.f};
-#pragma unroll
-  for (int k2 = 0; k2 < 4; k2++) {  // columns 8 k2 .. 8 k2 + 7
-    half8 hv, lv;
-#pragma unroll
-    for (int p = 0; p < 2; p++) {
-      const int k = 2 * k2 + p;  // columns 4k .. 4k + 3
-      const uint32_t l = realign(r.ql, k, r.shl), h = realign(r.qh, k, r.shh);
-      const uint32_t lo4 = (quarter < 2 ? l : l >> 4) & 0x0f0f0f0fu;
-      const uint32_t hi2 = (h >> (2 * quarter)) & 0x03030303u;
-      const uint32_t q = lo4 | (hi2 << 4);  // four 6-bit codes, a byte each
-      const uint32_t pa = (q & 0xffu) | ((q << 8) & 0xff0000u) | 0x64006400u;
-      const uint32_t pb = ((q >> 16) & 0xffu) | ((q >> 8) & 0xff0000u) | 0x64006400u;
-      const f16 sc = k < 4 ? s0 : s1;
-      const half2v scv = {sc, sc};
-      const half2v xa = __builtin_bit_cast(half2v, pa) + off, xb = __builtin_bit_cast(half2v, pb) + off;
-      const half2v ha = xa * scv, hb = xb * scv;
-      const half2v la = __builtin_elementwise_fma(xa, scv, -ha), lb = __builtin_elementwise_fma(xb, scv, -hb);
-      hv[4 * p] = ha[0];
-      hv[4 * p + 1] = ha[1];
-      hv[4 * p + 2] = hb[0];
-      hv[4 * p + 3] = hb[1];
-      lv[4 * p] = la[0];
-      lv[4 * p + 1] = la[1];
-      lv[4 * p + 2] = lb[0];
-      lv[4 * p + 3] = lb[1];
-    }
-    *reinterpret_cast<half8 *>(ws + 8 * k2) = hv;
-    *reinterpret_cast<half8 *>(wl + 8 * k2) = lv;
-  }
-}
-
 // The same tile, products and LDS layout with eight waves, so that two
 // workgroups per CU put four waves on each SIMD (the four-wave kernel's two
 // leave the matrix cores waiting on the staging chain's latency).  Waves 0-3
@@ -414,20 +353,16 @@ __device__ __forceinline__ void stage_q6k_codes(const Deq<LLRS_Q6_K>::Raw &r, in
 // to 128 registers.  Each output is the same sequence of MFMAs as in the
 // four-wave kernel.  Measured 4-5% faster per product (7B shape, 512
 // tokens); LLRS_PREFILL_GEMM=4 selects the four-wave kernel.
-template <uint32_t TY, int BM, bool CODES>
+template <uint32_t TY, int BM>
 __global__ __launch_bounds__(512) void prefill_gemm8_kernel(PrefillGemmArgs g) {
-  static_assert(!CODES || TY == LLRS_Q6_K, "integer-code staging is written for Q6_K");
   constexpr int MI = BM / 32;    // 16-token MFMA blocks per wave (BM/2 tokens)
   constexpr int NJ = 2;          // 16-row MFMA blocks per wave (32 rows)
   constexpr int APT = BM / 4;    // activation halves per staging thread and plane
   constexpr int TPR = 64 / APT;  // staging threads per activation row
   extern __shared__ __align__(16) f16 lds[];
   f16 *As = lds, *Al = As + BM * LS, *Ws = Al + BM * LS, *Wl = Ws + BN * LS;
-  // CODES: per weight row, the rescale of the current 256-column block and the current unit.
-  float *ratio = reinterpret_cast<float *>(Wl + BN * LS), *unit = ratio + BN;
   const int n0 = blockIdx.x * BN, t0 = blockIdx.y * BM;
-  const int per = CODES ? ((g.k >> 8) + g.ksplit - 1) / g.ksplit * 256
-                        : ((g.k + KC - 1) / KC + g.ksplit - 1) / g.ksplit * KC;
+  const int per = ((g.k + KC - 1) / KC + g.ksplit - 1) / g.ksplit * KC;
   const int kb = blockIdx.z * per, ke = min(g.k, kb + per);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;  // BM/2 tokens x 32 rows
@@ -460,21 +395,11 @@ __global__ __launch_bounds__(512) void prefill_gemm8_kernel(PrefillGemmArgs g) {
       }
     }
   };
-  float u = 1.f;  // CODES: a row's current unit (kept by its wc == 0 staging thread)
   if (kb < ke) load_chunk(kb);
   for (int k0 = kb; k0 < ke; k0 += KC) {
-    const int kc = min(KC, ke - k0);  // 32 or 64 (64 with CODES)
+    const int kc = min(KC, ke - k0);  // 32 or 64
     __syncthreads();  // the previous chunk's MFMAs have read LDS
-    bool staged = false;
-    if constexpr (CODES) {
-      if (wstage) {
-        stage_q6k_codes(pre.raw, k0 + wc, w_ok, (k0 & 255) == 0 && wc == 0, u, ratio + wr, unit + wr,
-                        Ws + wr * LS + wc, Wl + wr * LS + wc);
-        staged = true;
-      }
-    }
-    if (staged) {
-    } else if (wstage) {
+    if (wstage) {
       float v[32];
       Deq<TY>::decode(pre.raw, min(k0 + wc, ke - 32), v);  // the columns load_chunk read
       const bool in = w_ok && wc < kc;
@@ -502,14 +427,6 @@ __global__ __launch_bounds__(512) void prefill_gemm8_kernel(PrefillGemmArgs g) {
     }
     __syncthreads();
     if (k0 + KC < ke) load_chunk(k0 + KC);  // in flight during the MFMAs below
-    if (CODES && (k0 & 255) == 0) {
-#pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        const float r = ratio[wn * 32 + 16 * j + (lane & 15)];
-#pragma unroll
-        for (int i = 0; i < MI; i++) acc[i][j] *= r;
-      }
-    }
     for (int ks = 0; ks < kc; ks += 32) {
       half8 af[MI], al[MI], bf[NJ], bl[NJ];
 #pragma unroll
@@ -535,338 +452,9 @@ __global__ __launch_bounds__(512) void prefill_gemm8_kernel(PrefillGemmArgs g) {
         }
     }
   }
-  if (CODES && kb < ke) {
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-      const float d = unit[wn * 32 + 16 * j + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < MI; i++) acc[i][j] *= d;
-    }
-  }
   store_tile<MI, NJ>(g, acc, n0 + wn * 32, t0 + wm * (BM / 2), lane);
 }
 
-
-// The epilogue of a dual gate/up tile without split K: the waves of the up
-// row group (wn = 1) hand their accumulators to the waves of the gate row group
-// with the same tokens through LDS (the same lane and register layout), and
-// those write silu(g) * u as f16 pairs -- the arithmetic of swiglu_f16_kernel,
-// so the values are the same as the separate products followed by it -- and,
-// with xso, the 32-column sums of hi + lo (two 16-row blocks of a lane's
-// column group, reduced over the 16 lanes of each token quad).
-template <int MI, int NJ>
-__device__ __forceinline__ void swiglu_tile(const PrefillGemmArgs &g, const f32x4 (&acc)[MI][NJ], float *xch,
-                                            int wm, int wn, int tb, int lane) {
-#pragma clang fp contract(off)
-  __syncthreads();  // every wave is done with the LDS tiles
-  float *slot = xch + (size_t)wm * (MI * NJ * 4 * 64);
-  if (wn == 1) {
-#pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-      for (int j = 0; j < NJ; j++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) slot[((i * NJ + j) * 4 + e) * 64 + lane] = acc[i][j][e];
-  }
-  __syncthreads();
-  if (wn != 0) return;
-  const int f0 = blockIdx.x * 64;  // the tile's first gate/up row
-#pragma unroll
-  for (int i = 0; i < MI; i++) {
-    float xsum[NJ / 2][4];
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-      const int f = f0 + 16 * j + (lane & 15);
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int t = tb + 16 * i + 4 * (lane >> 4) + e;
-        const float x = acc[i][j][e], u = slot[((i * NJ + j) * 4 + e) * 64 + lane];
-        f16 hi = 0, lo = 0;
-        if (f < g.dual_rows && t < g.t) {
-          split_f16((x / (1.0f + expf(-x))) * u, hi, lo);
-          g.h[(size_t)t * g.ldh + f] = hi;
-          g.hl[(size_t)t * g.ldh + f] = lo;
-        }
-        const float v = (float)hi + (float)lo;
-        if (j % 2 == 0) xsum[j / 2][e] = v;
-        else xsum[j / 2][e] += v;
-      }
-    }
-    if (g.xso) {
-#pragma unroll
-      for (int q = 0; q < NJ / 2; q++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          float v = xsum[q][e];
-#pragma unroll
-          for (int b = 1; b < 16; b <<= 1) v += lane_partner(v, b);
-          const int t = tb + 16 * i + 4 * (lane >> 4) + e, f = f0 + 32 * q;
-          if ((lane & 15) == 0 && t < g.t && f < g.dual_rows)
-            split_f16(v, g.xso[(size_t)t * g.ldxso + (f >> 5)], g.xso_lo[(size_t)t * g.ldxso + (f >> 5)]);
-        }
-    }
-  }
-}
-
-// The Q4_K product with the weight codes as exact f16 integers.  A Q4_K
-// weight is d * sc * q - dmin * m (value_at, src/quant.rs:349-456): q < 16 per
-// column, sc and m < 64 per 32-column sub-block s, d and dmin per 256-column
-// super-block b.  sc * q <= 945 is an exact f16, so
-//   y = sum_b d_b * sum_{j in b} (sc q)_j x_j  -  sum_s (dmin m)_s * xsum_s
-// with xsum_s the sum of the activations over sub-block s.  The first sum is
-// an MFMA product of one exact weight plane with the activations' hi and lo
-// planes: two MFMAs where an f32 weight (hi + lo) needs three, and half the
-// weight staging and LDS traffic.  Its accumulators are kept in units of the
-// row's current d: at each super-block they are scaled by d_prev / d_b (a
-// super-block with d = 0 contributes nothing and keeps the unit), and by the
-// last d at the end.  The second sum is a K/32-long product of -dmin * m (an
-// exact f32, as hi + lo) with xsum (hi + lo, xsum_f16_kernel), run after the
-// first on the same tile, LDS and accumulators, three MFMAs per step.  The
-// layout, roles and tiles are those of prefill_gemm8_kernel; K splits into
-// whole super-blocks.  Integer and f16 arithmetic on the codes is exact, so
-// the result differs from the f32 weights' only in f32 rounding.
-template <int BM, int TG, bool DUAL>
-__global__ __launch_bounds__(512) void prefill_gemm_k4_kernel(PrefillGemmArgs g) {
-  static_assert(!DUAL || TG == 4, "dual tiles pair the two row groups of waves");
-  // TG token groups x 8/TG row groups of waves: a wave multiplies TW tokens x RW rows.
-  constexpr int TW = BM / TG, RW = BN * TG / 8, MI = TW / 16, NJ = RW / 16;
-  constexpr int APT = BM / 4, TPR = 64 / APT;
-  extern __shared__ __align__(16) f16 lds[];
-  f16 *As = lds, *Al = As + BM * LS, *Ws = Al + BM * LS, *Wl = Ws + BN * LS;
-  // Per weight row of the tile: the rescale of the current super-block and the current unit.
-  float *ratio = reinterpret_cast<float *>(Wl + BN * LS), *unit = ratio + BN;
-  const int n0 = blockIdx.x * BN, t0 = blockIdx.y * BM;
-  const int per = ((g.k >> 8) + g.ksplit - 1) / g.ksplit * 256;
-  const int kb = blockIdx.z * per, ke = min(g.k, kb + per);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave % TG, wn = wave / TG;
-  const bool wstage = wave < 4;
-  const int st = tid & 255;
-  f32x4 acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; i++)
-#pragma unroll
-    for (int j = 0; j < NJ; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int ar = st / TPR, ac = (st % TPR) * APT;
-  const int wr = st >> 1, wc = (st & 1) * 32;
-  // A segmented product: this tile's segment (boundaries are tile multiples).
-  const int seg = g.nseg > 1 ? (n0 >= g.seg_base[1]) + (g.nseg > 2 && n0 >= g.seg_base[2]) : 0;
-  const int sbase = g.nseg > 0 ? g.seg_base[seg] : 0;
-  const int srows = g.nseg > 0 ? g.seg_base[seg + 1] - sbase : g.n;
-  const uint8_t *wmat = g.nseg > 0 ? g.seg_w[seg] : g.w;
-  // DUAL: tile rows 0-63 are gate rows blockIdx.x * 64 + wr, rows 64-127 the same up rows.
-  const int wrow_i = DUAL ? blockIdx.x * 64 + (wr & 63) : n0 - sbase + wr;
-  const bool a_ok = t0 + ar < g.t, w_ok = wrow_i < (DUAL ? g.dual_rows : srows);
-  const int arow = a_ok ? t0 + ar : 0;
-  const uint8_t *wrow = (DUAL && wr >= 64 ? g.w2 : wmat) + (size_t)(w_ok ? wrow_i : 0) * g.row_bytes;
-  union Pre {
-    struct { half8 ah[APT / 8], al[APT / 8]; } a;
-    struct { uint4 hdr, q0, q1; } w;  // d, dmin, 12 scale bytes; the sub-block pair's 32 code bytes
-    uint4 mh[4];                      // the headers of four super-blocks (second sum)
-  } pre;
-
-  // ---- First sum: the exact codes, rescaled per super-block ----
-  auto load_codes = [&](int k0) {  // k0: a multiple of 64 with k0 + 64 <= ke
-    if (wstage) {
-      const uint8_t *b = wrow + (size_t)(k0 >> 8) * 144;
-      const int pair = (k0 & 255) >> 6;
-      pre.w.hdr = *reinterpret_cast<const uint4 *>(b);
-      pre.w.q0 = *reinterpret_cast<const uint4 *>(b + 16 + pair * 32);
-      pre.w.q1 = *reinterpret_cast<const uint4 *>(b + 32 + pair * 32);
-    } else {
-      const size_t o = (size_t)arow * g.lda + k0 + ac;
-#pragma unroll
-      for (int h = 0; h < APT / 8; h++) {
-        pre.a.ah[h] = *reinterpret_cast<const half8 *>(g.a + o + 8 * h);
-        pre.a.al[h] = *reinterpret_cast<const half8 *>(g.a_lo + o + 8 * h);
-      }
-    }
-  };
-  float u = 1.f;  // a row's current unit (kept by its wc == 0 staging thread)
-  if (kb < ke) load_codes(kb);
-  for (int k0 = kb; k0 < ke; k0 += KC) {
-    __syncthreads();  // the previous chunk's MFMAs have read LDS
-    if (wstage) {
-      const int sub = ((k0 + wc) & 255) >> 5;  // sub < 4 is uniform: k0 is
-      const uint32_t s[3] = {pre.w.hdr.y, pre.w.hdr.z, pre.w.hdr.w};
-      const int sc = sub < 4 ? (byte_of(s, sub) & 63)
-                             : ((byte_of(s, sub + 4) & 0x0f) | ((byte_of(s, sub - 4) >> 6) << 4));
-      const float d = f16_bits_to_f32((uint16_t)(pre.w.hdr.x & 0xffff));
-      const bool live = d != 0.f;  // NaN d is live and makes the row NaN, as in f32
-      if ((k0 & 255) == 0 && wc == 0) {
-        ratio[wr] = live ? u / d : 1.f;
-        if (live) u = d;
-        unit[wr] = u;
-      }
-      // (1024 + q) from the f16 bit pattern 0x6400 | q, then (1024 + q) * sc -
-      // 1024 * sc = sc * q, exact in one fma.
-      const f16 sch = (f16)(float)((w_ok && live) ? sc : 0);
-      const half2v f = {sch, sch}, c = {(f16)(-1024.f * (float)sch), (f16)(-1024.f * (float)sch)};
-      const uint32_t w[8] = {pre.w.q0.x, pre.w.q0.y, pre.w.q0.z, pre.w.q0.w,
-                             pre.w.q1.x, pre.w.q1.y, pre.w.q1.z, pre.w.q1.w};
-      const int shift = (sub & 1) * 4;
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        half8 h;
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-          const uint32_t v = (w[2 * q + p] >> shift) & 0x0f0f0f0fu;  // four codes, a byte each
-          const uint32_t lo = (v & 0xffu) | ((v << 8) & 0xff0000u) | 0x64006400u;
-          const uint32_t hi = ((v >> 16) & 0xffu) | ((v >> 8) & 0xff0000u) | 0x64006400u;
-          const half2v a = __builtin_elementwise_fma(__builtin_bit_cast(half2v, lo), f, c);
-          const half2v b = __builtin_elementwise_fma(__builtin_bit_cast(half2v, hi), f, c);
-          h[4 * p] = a[0];
-          h[4 * p + 1] = a[1];
-          h[4 * p + 2] = b[0];
-          h[4 * p + 3] = b[1];
-        }
-        *reinterpret_cast<half8 *>(Ws + wr * LS + wc + 8 * q) = h;
-      }
-    } else {
-      const half8 z = half8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-      for (int h = 0; h < APT / 8; h++) {
-        *reinterpret_cast<half8 *>(As + ar * LS + ac + 8 * h) = a_ok ? pre.a.ah[h] : z;
-        *reinterpret_cast<half8 *>(Al + ar * LS + ac + 8 * h) = a_ok ? pre.a.al[h] : z;
-      }
-    }
-    __syncthreads();
-    if (k0 + KC < ke) load_codes(k0 + KC);  // in flight during the MFMAs below
-    if ((k0 & 255) == 0) {
-#pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        const float r = ratio[wn * RW + 16 * j + (lane & 15)];
-#pragma unroll
-        for (int i = 0; i < MI; i++) acc[i][j] *= r;
-      }
-    }
-#pragma unroll
-    for (int ks = 0; ks < KC; ks += 32) {
-      half8 af[MI], al[MI], bf[NJ];
-#pragma unroll
-      for (int i = 0; i < MI; i++) {
-        const int o = (wm * TW + 16 * i + (lane & 15)) * LS + ks + 8 * (lane >> 4);
-        af[i] = *reinterpret_cast<const half8 *>(As + o);
-        al[i] = *reinterpret_cast<const half8 *>(Al + o);
-      }
-#pragma unroll
-      for (int j = 0; j < NJ; j++)
-        bf[j] = *reinterpret_cast<const half8 *>(Ws + (wn * RW + 16 * j + (lane & 15)) * LS + ks +
-                                                 8 * (lane >> 4));
-#pragma unroll
-      for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], bf[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
-        }
-    }
-  }
-  if (kb < ke) {
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-      const float d = unit[wn * RW + 16 * j + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < MI; i++) acc[i][j] *= d;
-    }
-  }
-
-  // ---- Second sum: - (dmin m)_s * xsum_s over this range's sub-blocks ----
-  const int mb = kb >> 5, me = ke >> 5;  // multiples of 8
-  auto load_mins = [&](int m0) {
-    if (wstage) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int s0 = m0 + wc + 8 * i;
-        pre.mh[i] = s0 < me ? *reinterpret_cast<const uint4 *>(wrow + (size_t)(s0 >> 3) * 144)
-                            : uint4{0, 0, 0, 0};
-      }
-    } else {
-      // Columns up to m0 + 64 <= K/32 + 56 < ldxs: in the buffer; those past
-      // the range are zeroed below.
-      const size_t o = (size_t)arow * g.ldxs + m0 + ac;
-#pragma unroll
-      for (int h = 0; h < APT / 8; h++) {
-        pre.a.ah[h] = *reinterpret_cast<const half8 *>(g.xs + o + 8 * h);
-        pre.a.al[h] = *reinterpret_cast<const half8 *>(g.xs_lo + o + 8 * h);
-      }
-    }
-  };
-  if (mb < me) load_mins(mb);
-  for (int m0 = mb; m0 < me; m0 += KC) {
-    const int mc = min(KC, me - m0);  // a multiple of 8
-    __syncthreads();
-    if (wstage) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const bool in = w_ok && m0 + wc + 8 * i < me;
-        const float dmin = f16_bits_to_f32((uint16_t)(pre.mh[i].x >> 16));
-        const uint32_t s[3] = {pre.mh[i].y, pre.mh[i].z, pre.mh[i].w};
-        half8 h, l;
-#pragma unroll
-        for (int e = 0; e < 8; e++) {  // scale_min_k4 (src/quant.rs:338-347), the m half
-          const int m = e < 4 ? (byte_of(s, e + 4) & 63) : ((byte_of(s, e + 4) >> 4) | ((byte_of(s, e) >> 6) << 4));
-          f16 a, b;
-          split_f16(in ? -(dmin * (float)m) : 0.f, a, b);
-          h[e] = a;
-          l[e] = b;
-        }
-        *reinterpret_cast<half8 *>(Ws + wr * LS + wc + 8 * i) = h;
-        *reinterpret_cast<half8 *>(Wl + wr * LS + wc + 8 * i) = l;
-      }
-    } else {
-      const half8 z = half8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-      for (int h = 0; h < APT / 8; h++) {
-        const bool in = a_ok && ac + 8 * h < mc;
-        *reinterpret_cast<half8 *>(As + ar * LS + ac + 8 * h) = in ? pre.a.ah[h] : z;
-        *reinterpret_cast<half8 *>(Al + ar * LS + ac + 8 * h) = in ? pre.a.al[h] : z;
-      }
-    }
-    __syncthreads();
-    if (m0 + KC < me) load_mins(m0 + KC);
-    for (int ks = 0; ks < mc; ks += 32) {
-      half8 af[MI], al[MI], bf[NJ], bl[NJ];
-#pragma unroll
-      for (int i = 0; i < MI; i++) {
-        const int o = (wm * TW + 16 * i + (lane & 15)) * LS + ks + 8 * (lane >> 4);
-        af[i] = *reinterpret_cast<const half8 *>(As + o);
-        al[i] = *reinterpret_cast<const half8 *>(Al + o);
-      }
-#pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        const int o = (wn * RW + 16 * j + (lane & 15)) * LS + ks + 8 * (lane >> 4);
-        bf[j] = *reinterpret_cast<const half8 *>(Ws + o);
-        bl[j] = *reinterpret_cast<const half8 *>(Wl + o);
-      }
-#pragma unroll
-      for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], bf[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bl[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
-        }
-    }
-  }
-  if constexpr (DUAL) {
-    if (g.ksplit == 1) {
-      swiglu_tile<MI, NJ>(g, acc, reinterpret_cast<float *>(lds), wm, wn, t0 + wm * TW, lane);
-      return;
-    }
-  }
-  if (g.nseg > 0 && g.ksplit == 1) {  // the segment's own output
-    PrefillGemmArgs gs = g;
-    gs.c = g.seg_c[seg];
-    gs.ldc = g.seg_ldc[seg];
-    gs.bias = g.seg_bias[seg];
-    gs.n = srows;
-    store_tile<MI, NJ>(gs, acc, n0 - sbase + wn * RW, t0 + wm * TW, lane);
-    return;
-  }
-  store_tile<MI, NJ>(g, acc, n0 + wn * RW, t0 + wm * TW, lane);
-}
 
 // xs + xs_lo [t][s] = the sum over j < 32 of a[t][32 s + j] + a_lo[t][32 s + j]
 // (in that order, in f32), as an f16 pair, for s < nsub.
@@ -1476,32 +1064,11 @@ void launch_tiles(const PrefillGemmArgs &a, int bm, hipStream_t s) {
   const dim3 grid((unsigned)((a.n + BN - 1) / BN), (unsigned)((a.t + bm - 1) / bm), (unsigned)a.ksplit);
   const size_t lds = (size_t)2 * (bm + BN) * LS * sizeof(f16);
   const bool w8 = eight_waves();
-  if (a.type == LLRS_Q4_K && a.xs) {
-    const size_t lds4 = lds + 2 * BN * sizeof(float);
-    if (a.w2 && bm == 128)
-      hipLaunchKernelGGL((prefill_gemm_k4_kernel<128, 4, true>), grid, dim3(512), lds4, s, a);
-    else if (a.w2)
-      hipLaunchKernelGGL((prefill_gemm_k4_kernel<64, 4, true>), grid, dim3(512), lds4, s, a);
-    else if (bm == 128)
-      hipLaunchKernelGGL((prefill_gemm_k4_kernel<128, 4, false>), grid, dim3(512), lds4, s, a);
-    else
-      hipLaunchKernelGGL((prefill_gemm_k4_kernel<64, 4, false>), grid, dim3(512), lds4, s, a);
-    return;
-  }
-
-  if (a.type == LLRS_Q6_K && w8 && prefill_codes_enabled()) {
-    const size_t lds6 = lds + 2 * BN * sizeof(float);
-    if (bm == 128)
-      hipLaunchKernelGGL((prefill_gemm8_kernel<LLRS_Q6_K, 128, true>), grid, dim3(512), lds6, s, a);
-    else
-      hipLaunchKernelGGL((prefill_gemm8_kernel<LLRS_Q6_K, 64, true>), grid, dim3(512), lds6, s, a);
-    return;
-  }
 #define GEMM8(T)                                                                           \
   if (bm == 128)                                                                           \
-    hipLaunchKernelGGL((prefill_gemm8_kernel<T, 128, false>), grid, dim3(512), lds, s, a); \
+    hipLaunchKernelGGL((prefill_gemm8_kernel<T, 128>), grid, dim3(512), lds, s, a); \
   else                                                                                     \
-    hipLaunchKernelGGL((prefill_gemm8_kernel<T, 64, false>), grid, dim3(512), lds, s, a);
+    hipLaunchKernelGGL((prefill_gemm8_kernel<T, 64>), grid, dim3(512), lds, s, a);
 #define GEMM4(T)                                                                       \
   if (bm == 128)                                                                       \
     hipLaunchKernelGGL((prefill_gemm_kernel<T, 128>), grid, dim3(256), lds, s, a);     \
@@ -1531,8 +1098,9 @@ void launch_tiles(const PrefillGemmArgs &a, int bm, hipStream_t s) {
 #undef GEMM8
 }
 
-// The tiles of `a` with K split over `ksplit` workgroups, then the
-// fixed-order reduction of their partials into C.
+// The tiles of `a` (bm tokens each; -r: register-decoded, r row waves a group) with K
+// split over `ksplit` workgroups, then the fixed-order reduction of their
+// partials into C.
 int launch_split(PrefillGemmArgs a, int bm, int ksplit, hipStream_t s) {
   a.ksplit = ksplit;
   if (ksplit > 1) {
@@ -1540,7 +1108,10 @@ int launch_split(PrefillGemmArgs a, int bm, int ksplit, hipStream_t s) {
       return set_error(LLRS_E_INVALID, "prefill GEMM: split-K scratch of %zu floats is too small (%d x %d x %d)",
                        a.part_cap, ksplit, a.t, a.n);
   }
-  launch_tiles(a, bm, s);
+  if (bm > 0)
+    launch_tiles(a, bm, s);
+  else
+    launch_prefill_reg(a, -bm, s);
   if (ksplit > 1 && a.w2)
     hipLaunchKernelGGL(split_reduce_swiglu_kernel, dim3((unsigned)((a.dual_rows + 255) / 256), (unsigned)a.t),
                        dim3(256), 0, s, a.part, a.n, a.t, ksplit, a.dual_rows, a.h, a.hl, a.ldh, a.xso, a.xso_lo,
@@ -1582,6 +1153,107 @@ int launch_xsum_f16(const f16 *a, const f16 *a_lo, int lda, int k, int T, f16 *x
   return LLRS_OK;
 }
 
+// Whether a product of 16-bit weights (nothing to decode) is better off with the
+// LDS-staged kernel's 128-token tiles: from 16 of a row wave's tiles (32 rows x up
+// to 64 tokens) a CU (four layers of the 7B shape in BF16, 900 tokens: 6,145
+// against 7,326 us; of 1.5B in F16, 900: 2,574 against 2,045).
+static bool many_half_tiles(uint32_t type, int rows, int t) {
+  if (type != LLRS_F16 && type != LLRS_BF16) return false;
+  const int tt = prefill_reg_token_tile(type, t);
+  return (long)((rows + 31) / 32) * ((t + tt - 1) / tt) >= 8L * gemm_slots();
+}
+
+bool prefill_fuses(uint32_t type, size_t row_bytes, int rows, int t) {
+  if (!prefill_codes_enabled() || !prefill_reg_supports(type)) return false;
+  if ((uint64_t)row_bytes * (uint64_t)rows >= 1ull << 32) return false;  // its rows' offsets are 32-bit words
+  return !many_half_tiles(type, rows, t);
+}
+
+// The rows of `g` from `from` on (a multiple of 64 of a dual product's gate
+// rows), `rows` of them (of each matrix).
+static PrefillGemmArgs rows_of(const PrefillGemmArgs &g, int from, int rows) {
+  PrefillGemmArgs r = g;
+  r.w = g.w + (size_t)from * (size_t)g.row_bytes;
+  if (g.w2) {
+    r.w2 = g.w2 + (size_t)from * (size_t)g.row_bytes;
+    r.dual_rows = rows;
+    r.n = 2 * rows;
+    r.h = g.h + from;
+    r.hl = g.hl + from;
+    if (g.xso) {
+      r.xso = g.xso + from / 32;
+      r.xso_lo = g.xso_lo + from / 32;
+    }
+  } else {
+    r.n = rows;
+    r.c = g.c + from;
+    r.bias = g.bias ? g.bias + from : nullptr;
+  }
+  return r;
+}
+
+// Whether the many-token kernel takes a register-decoded product: past one
+// 64-token tile, unless its tiles neither fill three quarters of the slots nor
+// leave room to split K (7B gate/up over 128 tokens, 296 tiles of 512 slots:
+// 137 us against 112; over 256: 187 against 214).  Q6_K ffn_down of 7B over 128
+// tokens: 78 us against 96, q and k over 256: 31 against 35, over 128 equal.
+static bool takes_big(const PrefillGemmArgs &g) {
+  if (g.t <= 64 || g.type == LLRS_F16 || g.type == LLRS_BF16) return false;
+  const int tile = prefill_reg_big_row_tile(g.type, g.w2 != nullptr), rows = g.w2 ? g.dual_rows : g.n;
+  const long tiles = (long)((rows + tile - 1) / tile) * ((g.t + 63) / 64), slots = gemm_slots();
+  return 2 * tiles <= slots || 4 * tiles >= 3 * slots;
+}
+
+// Register-decoded products over many tokens, two workgroups a CU: whole rounds
+// of tiles run as they are; a last round that would fill at most half the
+// slots (or a product with fewer tiles than slots) splits K over them.
+static int launch_reg_big(const PrefillGemmArgs &g, hipStream_t s) {
+  const int slots = gemm_slots(), nb = (g.k + 255) / 256;
+  const int tile = prefill_reg_big_row_tile(g.type, g.w2 != nullptr), rows = g.w2 ? g.dual_rows : g.n;
+  const int nt = (rows + tile - 1) / tile, mt = (g.t + 63) / 64;
+  auto splits = [&](int tiles, int n) {
+    const int ks = std::max(1, std::min({slots / tiles, nb, (int)(g.part_cap / ((size_t)g.t * n))}));
+    const int per = (nb + ks - 1) / ks;
+    return (nb + per - 1) / per;
+  };
+  const int per_round = slots / mt;  // row tiles per round of slots
+  const int full = per_round > 0 && g.nseg == 0 ? nt / per_round * per_round : 0, rem = nt - full;
+  if (full > 0 && rem > 0 && rem * mt * 2 <= slots) {
+    PrefillGemmArgs m = rows_of(g, 0, full * tile);
+    m.ksplit = 1;
+    launch_prefill_reg(m, 0, s);
+    const PrefillGemmArgs r = rows_of(g, full * tile, rows - full * tile);
+    return launch_split(r, 0, splits(rem * mt, r.n), s);
+  }
+  return launch_split(g, 0, nt * mt < slots ? splits(nt * mt, g.n) : 1, s);
+}
+
+// The register-decoded products, one workgroup a CU.  Its row waves (1 to 5 a
+// group) and the K ranges (whole rounds of 512 columns) are those for which
+// the CUs' passes x (rounds x waves per SIMD + a start of two) come out least.
+static int launch_reg(const PrefillGemmArgs &g, hipStream_t s) {
+  const int cus = gemm_slots() / 2, nu = (g.k + 511) / 512;
+  const int tile = prefill_reg_row_tile(g.w2 != nullptr), tt = prefill_reg_token_tile(g.type, g.t);
+  const int rows = g.w2 ? g.dual_rows : g.n, mt = (g.t + tt - 1) / tt;
+  int best = INT_MAX, row_waves = 1, per = nu;
+  for (int rw = prefill_reg_max_row_waves(); rw >= 1; rw--) {
+    if (g.w2 && g.xso && rw % 2) continue;  // sums of 32 columns: pairs of waves
+    const int wgs = (rows + tile * rw - 1) / (tile * rw) * mt;
+    const int ks = std::max(1, std::min({cus / wgs, nu, (int)(g.part_cap / ((size_t)g.t * g.n))}));
+    const int rounds = (nu + ks - 1) / ks, passes = (wgs * ((nu + rounds - 1) / rounds) + cus - 1) / cus;
+    const int cost = passes * (rounds * ((rw + 2) / 2) + 2);
+    if (cost < best) {
+      best = cost;
+      row_waves = rw;
+      per = rounds;
+    }
+  }
+  // The kernel cuts ceil(blocks / ksplit) 256-column blocks a range; 2 per of
+  // them leave its last range short, never empty.
+  const int nb = (g.k + 255) / 256;
+  return launch_split(g, -row_waves, (nb + 2 * per - 1) / (2 * per), s);
+}
+
 int launch_prefill_gemm(const PrefillGemmArgs &g, hipStream_t s) {
   if (g.k % 32 || g.lda % 8 || g.n <= 0 || g.k <= 0 || g.t <= 0)
     return set_error(LLRS_E_UNSUPPORTED, "prefill GEMM shape %d x %d (lda %d) is not supported", g.n,
@@ -1589,9 +1261,20 @@ int launch_prefill_gemm(const PrefillGemmArgs &g, hipStream_t s) {
   if (g.xs && (g.type != LLRS_Q4_K || g.k % 256 || g.ldxs % 8 || g.ldxs < g.k / 32 + 56))
     return set_error(LLRS_E_UNSUPPORTED, "prefill GEMM: activation sums (ldxs %d) for a type %u product of %d columns",
                      g.ldxs, g.type, g.k);
-  if (g.w2 && (!g.xs || g.dual_rows <= 0 || g.dual_rows % 64 || g.n != 2 * g.dual_rows || !g.h || !g.hl ||
+  const bool reg = prefill_fuses(g.type, (size_t)g.row_bytes, g.n, g.t) && (g.type != LLRS_Q4_K || g.xs);
+  if (g.w2 && (!reg || g.dual_rows <= 0 || g.dual_rows % 64 || g.n != 2 * g.dual_rows || !g.h || !g.hl ||
                (g.xso && g.ldxso < g.dual_rows / 32)))
     return set_error(LLRS_E_UNSUPPORTED, "prefill GEMM: dual gate/up product of %d rows is not supported", g.dual_rows);
+  if (g.nseg > 0 && (!reg || g.nseg > 3 || g.seg_base[0] != 0 || g.seg_base[g.nseg] != g.n))
+    return set_error(LLRS_E_UNSUPPORTED, "prefill GEMM: segmented product of %d segments is not supported", g.nseg);
+  for (int i = 1; i < g.nseg; i++)
+    if (g.seg_base[i] % BN || g.seg_base[i] <= g.seg_base[i - 1])
+      return set_error(LLRS_E_UNSUPPORTED, "prefill GEMM: segment boundary %d is not a multiple of %d", g.seg_base[i], BN);
+  if (reg) {
+    LLRS_TRY(takes_big(g) ? launch_reg_big(g, s) : launch_reg(g, s));
+    LLRS_HIP(hipGetLastError());
+    return LLRS_OK;
+  }
   // 128-token tiles when there are enough of them (the dequantized weight
   // tile then serves twice the tokens), else 64.  Products with fewer tiles
   // than half the slots split K over up to 8 workgroups (at least 6 K chunks
@@ -1608,36 +1291,12 @@ int launch_prefill_gemm(const PrefillGemmArgs &g, hipStream_t s) {
   const int per_round = slots / mt;  // row tiles per round of slots
   const int full = (ks == 1 && per_round > 0) ? ntiles / per_round * per_round : 0;
   const int rem = ntiles - full;
-  if (g.nseg > 0 && (g.type != LLRS_Q4_K || !g.xs || g.nseg > 3 || g.seg_base[0] != 0 || g.seg_base[g.nseg] != g.n))
-    return set_error(LLRS_E_UNSUPPORTED, "prefill GEMM: segmented product of %d segments is not supported", g.nseg);
-  for (int i = 1; i < g.nseg; i++)
-    if (g.seg_base[i] % BN || g.seg_base[i] <= g.seg_base[i - 1])
-      return set_error(LLRS_E_UNSUPPORTED, "prefill GEMM: segment boundary %d is not a multiple of %d", g.seg_base[i], BN);
-  if (g.nseg == 0 && full > 0 && rem > 0 && rem * mt * 2 <= slots) {
-    PrefillGemmArgs m = g;
-    m.n = full * BN;
+  if (full > 0 && rem > 0 && rem * mt * 2 <= slots) {
+    PrefillGemmArgs m = rows_of(g, 0, full * BN);
     m.ksplit = 1;
-    if (g.w2) m.dual_rows = full * BN / 2;
     launch_tiles(m, bm, s);
-    PrefillGemmArgs r = g;
-    r.n = g.n - full * BN;
-    if (g.w2) {  // the remaining gate/up rows from full * 64 on
-      const size_t f = (size_t)full * BN / 2;
-      r.w = g.w + f * (size_t)g.row_bytes;
-      r.w2 = g.w2 + f * (size_t)g.row_bytes;
-      r.dual_rows = g.dual_rows - (int)f;
-      r.h = g.h + f;
-      r.hl = g.hl + f;
-      if (g.xso) {
-        r.xso = g.xso + f / 32;
-        r.xso_lo = g.xso_lo + f / 32;
-      }
-    } else {
-      r.w = g.w + (size_t)full * BN * (size_t)g.row_bytes;
-      r.c = g.c + (size_t)full * BN;
-      r.bias = g.bias ? g.bias + (size_t)full * BN : nullptr;
-    }
-    LLRS_TRY(launch_split(r, bm, std::max(1, std::min({8, slots / (rem * mt), chunks / 6})), s));
+    LLRS_TRY(launch_split(rows_of(g, full * BN, g.n - full * BN), bm,
+                          std::max(1, std::min({8, slots / (rem * mt), chunks / 6})), s));
   } else {
     LLRS_TRY(launch_split(g, bm, ks, s));
   }

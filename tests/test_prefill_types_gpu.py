@@ -34,13 +34,35 @@ def check(llrs, oracle, model, tmp_path, vocab, layers, n, seed):
 
 @pytest.mark.parametrize("n", [2, 65, 257], ids=["2", "65", "257"])
 @pytest.mark.parametrize("dtype", ["BF16", "F16", "F32"])
-def test_prefill_float_weights(llrs, backend, oracle, tmp_path, dtype, n):
+@pytest.mark.parametrize("staged", [False, True], ids=["default", "lds_staged"])
+def test_prefill_float_weights(llrs, backend, oracle, tmp_path, monkeypatch, dtype, n, staged):
     """Unquantized checkpoints: FFN matrices of 2,080 rows (sixteen 128-row
     tiles and a remainder), two tokens, one past a 64-token tile, one past
-    two 128-token tiles."""
+    two 128-token tiles; on the default route and on the LDS-staged kernel
+    that large 16-bit products take."""
+    if staged:
+        monkeypatch.setenv("LLRS_PREFILL_CODES", "f32")
     cfg = llrs.SynthConfig(hidden_size=256, intermediate_size=2080, num_attention_heads=4, num_key_value_heads=2,
                            num_hidden_layers=2, vocab_size=1000, max_position_embeddings=512, seed=51,
                            tie_word_embeddings=False)
     write_checkpoint(llrs, cfg, tmp_path / "ck", dtype)
     model = llrs.ModelLoader.load(tmp_path / "ck", backend)
     check(llrs, oracle, model, tmp_path, cfg.vocab_size, cfg.num_hidden_layers, n, 51 + n)
+
+
+@pytest.mark.parametrize("n", [2, 16, 17, 32, 33, 65, 130])
+@pytest.mark.parametrize("hidden,heads,ffn,recipe", [(512, 4, 2304, "Q4KM"), (512, 8, 2112, "Q4K"),
+                                                     (352, 11, 2112, "Q4KM"), (384, 6, 2112, "Q4K")],
+                         ids=["q4k_q8_q6k", "q4k_q5", "q5_q8_ragged_k", "q5"])
+def test_prefill_quantized_weights(llrs, backend, oracle, tmp_path, hidden, heads, ffn, recipe, n):
+    """The register-decoded products: 16-, 32- and 64-token tiles full, with one
+    token too many and with remainders; FFN rows that end inside a row tile
+    (2,112); rows of a 32-column remainder past whole steps (352, 2,112); an
+    odd number of 256-column blocks (2,304); q/k/v in segments and apart (352
+    is no multiple of 128)."""
+    cfg = llrs.SynthConfig(hidden_size=hidden, intermediate_size=ffn, num_attention_heads=heads,
+                           num_key_value_heads=heads if heads == 11 else 2, num_hidden_layers=2, vocab_size=500,
+                           max_position_embeddings=256, seed=57, tie_word_embeddings=False,
+                           recipe=getattr(llrs.LoadQuantization, recipe))
+    model = llrs.HipQwen2Model.synthetic(backend, cfg)
+    check(llrs, oracle, model, tmp_path, cfg.vocab_size, cfg.num_hidden_layers, n, 57 + n)
