@@ -104,8 +104,10 @@ struct llrs_kv {
   hipGraph_t graph[4] = {};
   hipGraphExec_t exec[4] = {};
   std::vector<void *> allocs;
-  // Multi-token prefill buffers (allocated on first use, pf_cap token rows).
+  // Multi-token prefill buffers (allocated on first use, pf_cap token rows;
+  // those that grow with the rows in pf_allocs).
   size_t pf_cap = 0;
+  std::vector<void *> pf_allocs;
   float *pf_x = nullptr, *pf_q = nullptr, *pf_k = nullptr, *pf_v = nullptr, *pf_g = nullptr,
         *pf_u = nullptr;
   llrs::f16 *pf_h = nullptr, *pf_hl = nullptr;  // GEMM inputs as f16 hi + lo pairs
@@ -1053,6 +1055,7 @@ static void free_kv(llrs_kv *kv) {
     if (kv->graph[i]) (void)hipGraphDestroy(kv->graph[i]);
   }
   for (void *p : kv->allocs) (void)hipFree(p);
+  for (void *p : kv->pf_allocs) (void)hipFree(p);
   if (kv->p_bar_uc) uc_release(kv->p_bar);
   if (kv->pinned) (void)hipHostFree(kv->pinned);
   delete kv;
@@ -1140,20 +1143,31 @@ static int stage_tokens(llrs_kv *kv, const uint32_t *tokens, size_t n, size_t po
   return LLRS_OK;
 }
 
-// Rows of one prefill chunk: bounds the prefill buffers (7B: ~114 MB).
-constexpr size_t kPrefillRows = 512;
+// Rows of one prefill chunk: bounds the prefill buffers (7B: 0.54 GB).  Longer
+// chunks fill the CUs better and split the cache rows to f16 less often: 4,000
+// tokens of 1.5B take 9.0 ms per four layers in chunks of 512, 6.4 in 2,048 and
+// 6.3 in 4,096, whose buffers are twice as large.
+constexpr size_t kPrefillRows = 2048;
 
 static bool prefill_tokenwise() {
   const char *e = getenv("LLRS_PREFILL_TOKENWISE");
   return e && *e && *e != '0';
 }
 
-static int prefill_buffers(llrs_kv *kv) {
-  if (kv->pf_cap) return LLRS_OK;
+// Buffers for chunks of up to n rows, in steps of 512: a longer prompt than any
+// before replaces them (after the stream has finished with the old ones).
+static int prefill_buffers(llrs_kv *kv, size_t n) {
+  const size_t T = std::min({kv->max_seq_len, kPrefillRows, (n + 511) / 512 * 512});
+  if (kv->pf_cap >= T) return LLRS_OK;
   const llrs_model_config &c = kv->m->cfg;
-  const size_t T = kv->max_seq_len < kPrefillRows ? kv->max_seq_len : kPrefillRows;
   const size_t H = c.hidden_size, F = c.intermediate_size, KV = c.kv_width;
-  auto A = [&](void **p, size_t bytes) { return dev_alloc(kv->allocs, p, bytes); };
+  if (!kv->pf_allocs.empty()) {
+    LLRS_HIP(hipStreamSynchronize(kv->m->b->stream));
+    kv->pf_cap = 0;
+    for (void *p : kv->pf_allocs) LLRS_HIP(hipFree(p));
+    kv->pf_allocs.clear();
+  }
+  auto A = [&](void **p, size_t bytes) { return dev_alloc(kv->pf_allocs, p, bytes); };
   LLRS_TRY(A((void **)&kv->pf_x, T * H * 4));
   LLRS_TRY(A((void **)&kv->pf_q, T * H * 4));
   LLRS_TRY(A((void **)&kv->pf_k, T * KV * 4));
@@ -1162,27 +1176,23 @@ static int prefill_buffers(llrs_kv *kv) {
   LLRS_TRY(A((void **)&kv->pf_u, T * F * 4));
   LLRS_TRY(A((void **)&kv->pf_h, T * (H > F ? H : F) * 2));
   LLRS_TRY(A((void **)&kv->pf_hl, T * (H > F ? H : F) * 2));
-  // Room for a Q4_K product's reads past the last sum (k/32 + 56 columns).
-  kv->pf_ldxs = (int)(((H > F ? H : F) / 32 + 56 + 7) / 8 * 8);
+  kv->pf_ldxs = (int)(((H > F ? H : F) / 32 + 7) / 8 * 8);
   LLRS_TRY(A((void **)&kv->pf_xs, T * kv->pf_ldxs * 2));
   LLRS_TRY(A((void **)&kv->pf_xsl, T * kv->pf_ldxs * 2));
   LLRS_TRY(A((void **)&kv->pf_xs2, T * kv->pf_ldxs * 2));
   LLRS_TRY(A((void **)&kv->pf_xsl2, T * kv->pf_ldxs * 2));
-  LLRS_HIP(hipMemset(kv->pf_xs, 0, T * kv->pf_ldxs * 2));
-  LLRS_HIP(hipMemset(kv->pf_xsl, 0, T * kv->pf_ldxs * 2));
-  LLRS_HIP(hipMemset(kv->pf_xs2, 0, T * kv->pf_ldxs * 2));
-  LLRS_HIP(hipMemset(kv->pf_xsl2, 0, T * kv->pf_ldxs * 2));
-  {
-    const size_t np = (kv->max_seq_len + 15) / 16 * 16, n = np * KV * 2;
+  if (!kv->pf_part) {
+    const size_t np = (kv->max_seq_len + 15) / 16 * 16, b = np * KV * 2;
     kv->pf_kvf.positions = (int)np;
     kv->pf_kvf.kvw = (int)KV;
-    LLRS_TRY(A((void **)&kv->pf_kvf.kh, n));
-    LLRS_TRY(A((void **)&kv->pf_kvf.kl, n));
-    LLRS_TRY(A((void **)&kv->pf_kvf.vh, n));
-    LLRS_TRY(A((void **)&kv->pf_kvf.vl, n));
+    auto K = [&](void **p, size_t bytes) { return dev_alloc(kv->allocs, p, bytes); };
+    LLRS_TRY(K((void **)&kv->pf_kvf.kh, b));
+    LLRS_TRY(K((void **)&kv->pf_kvf.kl, b));
+    LLRS_TRY(K((void **)&kv->pf_kvf.vh, b));
+    LLRS_TRY(K((void **)&kv->pf_kvf.vl, b));
+    kv->pf_part_cap = prefill_split_scratch_floats();
+    LLRS_TRY(K((void **)&kv->pf_part, kv->pf_part_cap * 4));
   }
-  kv->pf_part_cap = prefill_split_scratch_floats();
-  LLRS_TRY(A((void **)&kv->pf_part, kv->pf_part_cap * 4));
   kv->pf_cap = T;
   return LLRS_OK;
 }
@@ -1195,12 +1205,7 @@ static bool needs_xsum(std::initializer_list<const llrs_tensor *> ws) {
   return false;
 }
 
-// The activation sums of a/a_lo (k columns) that Q4_K products of this input read.
-static int prefill_xsum(llrs_kv *kv, const f16 *a, const f16 *a_lo, int k, int T, hipStream_t s) {
-  return launch_xsum_f16(a, a_lo, k, k, T, kv->pf_xs, kv->pf_xsl, kv->pf_ldxs, s);
-}
-
-// `xsum`: prefill_xsum has run on this input (Q4_K weights then take the integer-code product).
+// `xsum`: pf_xs holds this input's 32-column sums (Q4_K products read them).
 static int prefill_gemm(llrs_kv *kv, const llrs_tensor *w, const f16 *a, const f16 *a_lo, int lda,
                         float *c, int ldc, const float *bias, int T, bool accumulate, bool xsum,
                         hipStream_t s, bool xs2 = false) {
@@ -1330,7 +1335,7 @@ static int prefill_qkv_segmented(llrs_kv *kv, const DevLayer &L, int H, int KV, 
 static int prefill_batched(llrs_model *m, llrs_kv *kv, size_t start, size_t n) {
   const llrs_model_config &c = m->cfg;
   hipStream_t s = m->b->stream;
-  LLRS_TRY(prefill_buffers(kv));
+  LLRS_TRY(prefill_buffers(kv, n));
   const int H = (int)c.hidden_size, F = (int)c.intermediate_size, KV = (int)c.kv_width;
   const int nh = (int)c.num_attention_heads, nkv = (int)c.num_key_value_heads, hd = (int)c.head_dim;
   const float eps = c.rms_norm_eps, scale = 1.0f / sqrtf((float)hd);
@@ -1354,11 +1359,11 @@ static int prefill_batched(llrs_model *m, llrs_kv *kv, size_t start, size_t n) {
       }
       if (!with_v)
         LLRS_TRY(prefill_gemm(kv, L.v, kv->pf_h, kv->pf_hl, H, kv->pf_v, KV, L.bv, T, false, xs, s));
-      LLRS_TRY(launch_rope_append(kv->pf_q, kv->pf_k, kv->pf_v, kv->rope, T, st, nh, nkv, hd, kc, vc, s));
-      LLRS_TRY(launch_attention_rows(kv->pf_q, kc, vc, T, st, nh, nkv, hd, scale, kv->pf_h, kv->pf_hl, s,
-                                     &kv->pf_kvf));
+      LLRS_TRY(launch_rope_append(kv->pf_q, kv->pf_k, kv->pf_v, kv->rope, T, st, nh, nkv, hd, kc, vc, s,
+                                  &kv->pf_kvf));
       xs = needs_xsum({L.o});
-      if (xs) LLRS_TRY(prefill_xsum(kv, kv->pf_h, kv->pf_hl, H, T, s));
+      LLRS_TRY(launch_attention_rows(kv->pf_q, kc, vc, T, st, nh, nkv, hd, scale, kv->pf_h, kv->pf_hl, s,
+                                     &kv->pf_kvf, xs ? kv->pf_xs : nullptr, kv->pf_xsl, kv->pf_ldxs));
       LLRS_TRY(prefill_gemm(kv, L.o, kv->pf_h, kv->pf_hl, H, kv->pf_x, H, nullptr, T, true, xs, s));
       xs = needs_xsum({L.gate, L.up});
       LLRS_TRY(launch_rmsnorm_rows_f16(kv->pf_x, L.ffn_norm, kv->pf_h, kv->pf_hl, T, H, eps, s,

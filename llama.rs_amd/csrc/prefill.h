@@ -31,7 +31,7 @@ struct PrefillGemmArgs {
   float *part;
   size_t part_cap;  // floats
   // Q4_K weights: when set, the per-sub-block sums of the activations
-  // (launch_xsum_f16 of a/a_lo, [T][ldxs], ldxs >= k/32 + 56) and the product
+  // (launch_xsum_f16 of a/a_lo, [T][ldxs], ldxs >= k/32) and the product
   // runs on the Q4_K codes as exact integers (prefill_codes_enabled()).
   const f16 *xs, *xs_lo;
   int ldxs;
@@ -91,10 +91,6 @@ int launch_embed_rows(const llrs_tensor *emb, const uint32_t *tok, int T, float 
 // to f32 summation order).
 int launch_rmsnorm_rows_f16(const float *x, const float *w, f16 *out, f16 *out_lo, int T, int H,
                             float eps, hipStream_t s, f16 *xs = nullptr, f16 *xs_lo = nullptr, int ldxs = 0);
-// Split-half RoPE of q (in place) and k at positions start + t, and the K/V
-// cache rows of those positions.
-int launch_rope_append(float *q, const float *k, const float *v, const float *rope, int T, int start,
-                       int nh, int nkv, int hd, float *k_cache, float *v_cache, hipStream_t s);
 // Scratch for the f16 attention: one layer's K and V rows as hi/lo planes in
 // blocks of 16 positions (positions x kvw halves a plane; positions a
 // multiple of 16 and at least the rows attended, rounded up to 16).
@@ -102,13 +98,19 @@ struct PrefillKvF16 {
   f16 *kh, *kl, *vh, *vl;
   int positions, kvw;
 };
+// Split-half RoPE of q (in place) and k at positions start + t, and the K/V
+// cache rows of those positions.  With kvf (head_dim >= 32 and unless
+// LLRS_PREFILL_ATTN=f32) its planes then hold positions [0, start + T).
+int launch_rope_append(float *q, const float *k, const float *v, const float *rope, int T, int start,
+                       int nh, int nkv, int hd, float *k_cache, float *v_cache, hipStream_t s,
+                       const PrefillKvF16 *kvf);
 // Causal GQA attention of the T query rows (positions start + t) over the
-// cache, out + out_lo [T][nh*hd] (f16 pairs).  With kvf (head_dim >= 32 and
-// unless LLRS_PREFILL_ATTN=f32) the products run as f16 hi/lo MFMAs on a copy
-// of the cache rows in kvf; otherwise as f32 MFMAs on the cache.
+// cache, out + out_lo [T][nh*hd] (f16 pairs) and, with xs, their 32-column
+// sums.  With kvf (as for launch_rope_append, which fills it) the products run
+// as f16 hi/lo MFMAs on its planes; otherwise as f32 MFMAs on the cache.
 int launch_attention_rows(const float *q, const float *k_cache, const float *v_cache, int T,
                           int start, int nh, int nkv, int hd, float scale, f16 *out, f16 *out_lo,
-                          hipStream_t s, const PrefillKvF16 *kvf = nullptr);
+                          hipStream_t s, const PrefillKvF16 *kvf, f16 *xs, f16 *xs_lo, int ldxs);
 // out + out_lo [i] = silu(g[i]) * u[i] as f16 pairs, i < n (rows of `cols`);
 // with xs set, also their 32-column sums per row.
 int launch_swiglu_f16(const float *g, const float *u, f16 *out, f16 *out_lo, size_t n, int cols, hipStream_t s,

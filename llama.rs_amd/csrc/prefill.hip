@@ -494,88 +494,65 @@ __device__ __forceinline__ void half_wave_xsum(float v, int col, f16 *xs, f16 *x
   if ((threadIdx.x & 31) == 0) split_f16(v, xs[col >> 5], xs_lo[col >> 5]);
 }
 
-__global__ __launch_bounds__(256) void rmsnorm_rows_f16_kernel(const float *__restrict__ x,
-                                                               const float *__restrict__ w,
-                                                               f16 *__restrict__ out,
-                                                               f16 *__restrict__ out_lo, int H,
-                                                               float eps, f16 *__restrict__ xs,
-                                                               f16 *__restrict__ xs_lo, int ldxs) {
+// A thread holds eight consecutive columns (two 16-byte loads of x and of w, all
+// issued before the row's sum; one 16-byte store a plane), and four lanes a
+// 32-column sum.  One column a thread and pass chained the sums' exchanges 14
+// times over 3,584 columns: 10.0 us for 24 such rows, 6.0 this way.
+__global__ __launch_bounds__(1024) void rmsnorm_rows_f16_kernel(const float *__restrict__ x,
+                                                                const float *__restrict__ w,
+                                                                f16 *__restrict__ out,
+                                                                f16 *__restrict__ out_lo, int H,
+                                                                float eps, f16 *__restrict__ xs,
+                                                                f16 *__restrict__ xs_lo, int ldxs) {
 #pragma clang fp contract(off)
-  constexpr int kPer = 32;  // values a thread holds in registers (rows up to 8,192)
-  __shared__ float red[4];
-  const float *xr = x + (size_t)blockIdx.x * H;
-  const bool held = H <= kPer * 256;
-  float xv[kPer];
-  float s = 0.f;
-  if (held) {  // every load issued before the first is used
-#pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      const int i = k * 256 + threadIdx.x;
-      xv[k] = i < H ? xr[i] : 0.f;
-    }
-#pragma unroll
-    for (int k = 0; k < kPer; k++)
-      if (k * 256 + threadIdx.x < H) s += xv[k] * xv[k];
-  } else {
-    for (int i = threadIdx.x; i < H; i += 256) s += xr[i] * xr[i];
-  }
-  s = wave_total(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  const float tot = red[0] + red[1] + red[2] + red[3];
-  const float inv = 1.0f / sqrtf(tot / (float)H + eps);
-  f16 *o = out + (size_t)blockIdx.x * H, *ol = out_lo + (size_t)blockIdx.x * H;
-  auto emit = [&](int i, float xi) {  // i0 + threadIdx.x: whole passes, so the sums' shuffles see every lane
-    float v = 0.f;
-    if (i < H) {
-      f16 h, l;
-      split_f16(xi * (inv * w[i]), h, l);
-      o[i] = h;
-      ol[i] = l;
-      v = (float)h + (float)l;
-    }
-    if (xs && i - (int)(threadIdx.x & 31) < H)
-      half_wave_xsum(v, i, xs + (size_t)blockIdx.x * ldxs, xs_lo + (size_t)blockIdx.x * ldxs);
+  __shared__ float red[16];
+  const float4 *xr = reinterpret_cast<const float4 *>(x + (size_t)blockIdx.x * H), *wr = reinterpret_cast<const float4 *>(w);
+  const int G = H / 8, tid = threadIdx.x, nt = blockDim.x;
+  const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+  // The first group stays in registers (the whole row up to 8,192 columns).
+  const bool own = tid < G;
+  const float4 x0 = own ? xr[2 * tid] : z, x1 = own ? xr[2 * tid + 1] : z;
+  const float4 w0 = own ? wr[2 * tid] : z, w1 = own ? wr[2 * tid + 1] : z;
+  auto square = [](float4 a, float4 b) {
+    return a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w + b.x * b.x + b.y * b.y + b.z * b.z + b.w * b.w;
   };
-  if (held) {
+  float s = square(x0, x1);
+  for (int g = tid + nt; g < G; g += nt) s += square(xr[2 * g], xr[2 * g + 1]);
+  s = wave_total(s);
+  if ((tid & 63) == 0) red[tid >> 6] = s;
+  __syncthreads();
+  float tot = 0.f;
+  for (int i = 0; i < nt >> 6; i++) tot += red[i];
+  const float inv = 1.0f / sqrtf(tot / (float)H + eps);
+  auto emit = [&](int g, float4 a, float4 b, float4 u, float4 v) {  // every lane of a group of four takes part
+    const float xv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}, wv[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+    half8 h, l;
+    float sum = 0.f;
 #pragma unroll
-    for (int k = 0; k < kPer; k++)
-      if (k * 256 < H) emit(k * 256 + threadIdx.x, xv[k]);
-  } else {
-    for (int i0 = 0; i0 < H; i0 += 256) emit(i0 + threadIdx.x, i0 + threadIdx.x < H ? xr[i0 + threadIdx.x] : 0.f);
+    for (int e = 0; e < 8; e++) {
+      f16 hi, lo;
+      split_f16(xv[e] * (inv * wv[e]), hi, lo);
+      h[e] = hi;
+      l[e] = lo;
+      sum += (float)hi + (float)lo;
+    }
+    if (g < G) {
+      *reinterpret_cast<half8 *>(out + (size_t)blockIdx.x * H + 8 * g) = h;
+      *reinterpret_cast<half8 *>(out_lo + (size_t)blockIdx.x * H + 8 * g) = l;
+    }
+    if (xs) {
+      sum += lane_partner(sum, 1);
+      sum += lane_partner(sum, 2);
+      if ((g & 3) == 0 && g < G)
+        split_f16(sum, xs[(size_t)blockIdx.x * ldxs + (g >> 2)], xs_lo[(size_t)blockIdx.x * ldxs + (g >> 2)]);
+    }
+  };
+  emit(tid, x0, x1, w0, w1);
+  for (int g0 = nt; g0 < G; g0 += nt) {
+    const int g = g0 + tid;
+    const bool in = g < G;
+    emit(g, in ? xr[2 * g] : z, in ? xr[2 * g + 1] : z, in ? wr[2 * g] : z, in ? wr[2 * g + 1] : z);
   }
-}
-
-// Split-half RoPE (src/model.rs:87-95) of the row's query heads (in place)
-// and key heads, and the K/V cache rows of position start + t
-// (KVCache::update, src/cache.rs:38-53).
-__global__ __launch_bounds__(256) void rope_append_kernel(float *__restrict__ q,
-                                                          const float *__restrict__ k,
-                                                          const float *__restrict__ v,
-                                                          const float *__restrict__ rope, int start,
-                                                          int nh, int nkv, int hd,
-                                                          float *__restrict__ k_cache,
-                                                          float *__restrict__ v_cache) {
-  const int t = blockIdx.x, p = start + t, half = hd / 2, kvw = nkv * hd;
-  const float *cs = rope + (size_t)p * hd, *sn = cs + half;
-  float *qr = q + (size_t)t * nh * hd;
-  for (int i = threadIdx.x; i < nh * half; i += blockDim.x) {
-    const int h = i / half, j = i % half;
-    const float re = qr[h * hd + j], im = qr[h * hd + j + half];
-    qr[h * hd + j] = re * cs[j] - im * sn[j];
-    qr[h * hd + j + half] = re * sn[j] + im * cs[j];
-  }
-  const float *kr = k + (size_t)t * kvw;
-  float *kd = k_cache + (size_t)p * kvw;
-  for (int i = threadIdx.x; i < nkv * half; i += blockDim.x) {
-    const int h = i / half, j = i % half;
-    const float re = kr[h * hd + j], im = kr[h * hd + j + half];
-    kd[h * hd + j] = re * cs[j] - im * sn[j];
-    kd[h * hd + j + half] = re * sn[j] + im * cs[j];
-  }
-  const float *vr = v + (size_t)t * kvw;
-  float *vd = v_cache + (size_t)p * kvw;
-  for (int i = threadIdx.x; i < kvw; i += blockDim.x) vd[i] = vr[i];
 }
 
 // Causal GQA attention (src/model.rs:206-231, softmax_inplace 298-313) for a
@@ -780,6 +757,85 @@ __global__ __launch_bounds__(256) void kv_split_f16_kernel(const float *__restri
   }
 }
 
+// Split-half RoPE (src/model.rs:87-95) of 16 positions' rows of one head, by
+// absolute position: blockIdx.y a query head (in place), a key head (into the
+// cache, KVCache::update, src/cache.rs:38-53) or a value head (copied to the
+// cache).  With kh set, the new rows also go to the f16 planes that
+// kv_split_f16_kernel describes (earlier rows are its job), with zeros after the
+// last one in its block.  Sixteen lanes a position.  Bound by a launch's own
+// time: 5.1 us for 24 tokens of 28 + 4 heads of 128, where a workgroup a token
+// and a kv_split_f16_kernel over all rows after it took 5.4 + 4.4.
+template <int HD>
+__global__ __launch_bounds__(256) void rope_append_kernel(float *__restrict__ q, const float *__restrict__ k,
+                                                          const float *__restrict__ v,
+                                                          const float *__restrict__ rope, int T, int start, int nh,
+                                                          int nkv, float *__restrict__ k_cache,
+                                                          float *__restrict__ v_cache, f16 *__restrict__ kh,
+                                                          f16 *__restrict__ kl, f16 *__restrict__ vh,
+                                                          f16 *__restrict__ vl) {
+  constexpr int half = HD / 2, P = HD >= 32 ? HD / 32 : 1;  // pairs a lane
+  __shared__ float tile[16][HD + 1];
+  const int kvw = nkv * HD, y = blockIdx.y, c = threadIdx.x & 15, tl = threadIdx.x >> 4;
+  const int p0 = (start & ~15) + 16 * blockIdx.x, pos = p0 + tl, t = pos - start;
+  const bool in = t >= 0 && t < T;
+  if (y < nh + nkv) {
+    const bool is_q = y < nh;
+    const int d0 = (is_q ? y : y - nh) * HD;  // the head's first column
+    const float *src = is_q ? q + (size_t)t * nh * HD + d0 : k + (size_t)t * kvw + d0;
+    const float *cs = rope + (size_t)pos * HD, *sn = cs + half;
+#pragma unroll
+    for (int e = 0; e < P; e++) {
+      const int j = c * P + e;
+      if (HD == 16 && j >= half) continue;
+      float a = 0.f, b = 0.f;
+      if (in) {
+        const float re = src[j], im = src[j + half];
+        a = re * cs[j] - im * sn[j];
+        b = re * sn[j] + im * cs[j];
+        float *dst = is_q ? q + (size_t)t * nh * HD + d0 : k_cache + (size_t)pos * kvw + d0;
+        dst[j] = a;
+        dst[j + half] = b;
+      }
+      if (kh && !is_q && t >= 0) {
+        const size_t o = kblk_index(pos, d0 + j, kvw), o2 = kblk_index(pos, d0 + j + half, kvw);
+        split_f16(a, kh[o], kl[o]);
+        split_f16(b, kh[o2], kl[o2]);
+      }
+    }
+    return;
+  }
+  const int d0 = (y - nh - nkv) * HD;
+#pragma unroll
+  for (int e = 0; e < HD / 16; e++) {
+    const int d = c + 16 * e;
+    const float x = in ? v[(size_t)t * kvw + d0 + d] : 0.f;
+    if (in) v_cache[(size_t)pos * kvw + d0 + d] = x;
+    if (kh) tile[tl][d] = x;
+  }
+  if (!kh) return;
+  __syncthreads();
+  for (int i = threadIdx.x; i < 2 * HD; i += 256) {  // a dim's 16 positions in one plane: 32 contiguous bytes
+    const int d = i % HD;
+    f16 *plane = i < HD ? vh : vl;
+    half8 w[2];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      f16 hi, lo;
+      split_f16(tile[r][d], hi, lo);
+      w[r >> 3][r & 7] = i < HD ? hi : lo;
+    }
+    f16 *dst = plane + vblk_index(p0, d0 + d, kvw);
+    if (p0 >= start) {
+      reinterpret_cast<half8 *>(dst)[0] = w[0];
+      reinterpret_cast<half8 *>(dst)[1] = w[1];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+        if (p0 + r >= start) dst[r] = w[r >> 3][r & 7];
+    }
+  }
+}
+
 // attention_tile_kernel's tiles, order, online softmax and merge with f16
 // matrix products: q, K, V and the softmax weights as hi + lo pairs and three
 // MFMAs per product (hi*hi, hi*lo, lo*hi), accumulated in f32.  Scores: S^T =
@@ -796,7 +852,8 @@ __global__ __launch_bounds__(256, 3) void attention_f16_kernel(const float *__re
                                                             const f16 *__restrict__ vl,
                                                             const float *__restrict__ v_cache, int T,
                                                             int start, int nh, int nkv, float scale,
-                                                            f16 *__restrict__ out, f16 *__restrict__ out_lo) {
+                                                            f16 *__restrict__ out, f16 *__restrict__ out_lo,
+                                                            f16 *__restrict__ xs, f16 *__restrict__ xs_lo, int ldxs) {
   constexpr int NC = HD / 32;  // 32-dim score steps
   constexpr int NT = HD / 16;  // 16-dim output tiles
   __shared__ float so[4][16][HD + 4];
@@ -929,15 +986,33 @@ __global__ __launch_bounds__(256, 3) void attention_f16_kernel(const float *__re
   }
   const int p = start + q0 + qi;
   const size_t at = (size_t)(q0 + qi) * nh * HD + h * HD + c * NT;
+  float sum = 0.f;
+  auto emit = [&](int e, float v) {
+    f16 hi, lo;
+    split_f16(v, hi, lo);
+    out[at + e] = hi;
+    out_lo[at + e] = lo;
+    sum += (float)hi + (float)lo;
+  };
   if (isfinite(Lt) && Lt > 0.f) {
 #pragma unroll
-    for (int e = 0; e < NT; e++) split_f16(acc[e] / Lt, out[at + e], out_lo[at + e]);
+    for (int e = 0; e < NT; e++) emit(e, acc[e] / Lt);
   } else {
     const float *vp = v_cache + (size_t)kvh * HD + c * NT;
     for (int e = 0; e < NT; e++) {
       float vs = 0.f;
       for (int j = 0; j <= p; j++) vs += vp[(size_t)j * kvw + e];
-      split_f16(vs / (float)(p + 1), out[at + e], out_lo[at + e]);
+      emit(e, vs / (float)(p + 1));
+    }
+  }
+  // The output's 32-column sums, 32 / NT lanes of the query's 16: in a pass of
+  // their own (xsum_f16_kernel) they took 4.4 us for 24 tokens; nothing here.
+  if (xs) {
+#pragma unroll
+    for (int b = 1; b < 32 / NT; b <<= 1) sum += lane_partner(sum, b);
+    if (c % (32 / NT) == 0) {
+      const size_t o = (size_t)(q0 + qi) * ldxs + (h * HD + c * NT) / 32;
+      split_f16(sum, xs[o], xs_lo[o]);
     }
   }
 }
@@ -1258,7 +1333,7 @@ int launch_prefill_gemm(const PrefillGemmArgs &g, hipStream_t s) {
   if (g.k % 32 || g.lda % 8 || g.n <= 0 || g.k <= 0 || g.t <= 0)
     return set_error(LLRS_E_UNSUPPORTED, "prefill GEMM shape %d x %d (lda %d) is not supported", g.n,
                      g.k, g.lda);
-  if (g.xs && (g.type != LLRS_Q4_K || g.k % 256 || g.ldxs % 8 || g.ldxs < g.k / 32 + 56))
+  if (g.xs && (g.type != LLRS_Q4_K || g.k % 256 || g.ldxs % 8 || g.ldxs < g.k / 32))
     return set_error(LLRS_E_UNSUPPORTED, "prefill GEMM: activation sums (ldxs %d) for a type %u product of %d columns",
                      g.ldxs, g.type, g.k);
   const bool reg = prefill_fuses(g.type, (size_t)g.row_bytes, g.n, g.t) && (g.type != LLRS_Q4_K || g.xs);
@@ -1316,16 +1391,10 @@ int launch_rmsnorm_rows_f16(const float *x, const float *w, f16 *out, f16 *out_l
                             float eps, hipStream_t s, f16 *xs, f16 *xs_lo, int ldxs) {
   if (xs && (H % 32 || ldxs < H / 32))
     return set_error(LLRS_E_UNSUPPORTED, "activation sums over %d columns (ldxs %d)", H, ldxs);
-  hipLaunchKernelGGL(rmsnorm_rows_f16_kernel, dim3(T), dim3(256), 0, s, x, w, out, out_lo, H, eps, xs, xs_lo,
+  if (H % 8) return set_error(LLRS_E_UNSUPPORTED, "prefill RMSNorm over %d columns", H);
+  const int threads = std::min(1024, (H / 8 + 63) / 64 * 64);
+  hipLaunchKernelGGL(rmsnorm_rows_f16_kernel, dim3(T), dim3(threads), 0, s, x, w, out, out_lo, H, eps, xs, xs_lo,
                      ldxs);
-  LLRS_HIP(hipGetLastError());
-  return LLRS_OK;
-}
-
-int launch_rope_append(float *q, const float *k, const float *v, const float *rope, int T, int start,
-                       int nh, int nkv, int hd, float *k_cache, float *v_cache, hipStream_t s) {
-  hipLaunchKernelGGL(rope_append_kernel, dim3(T), dim3(256), 0, s, q, k, v, rope, start, nh, nkv, hd,
-                     k_cache, v_cache);
   LLRS_HIP(hipGetLastError());
   return LLRS_OK;
 }
@@ -1335,22 +1404,48 @@ bool prefill_attention_f16() {
   return !(e && strcmp(e, "f32") == 0);
 }
 
+static bool use_f16_planes(const PrefillKvF16 *kvf, int hd) { return kvf && hd >= 32 && prefill_attention_f16(); }
+
+int launch_rope_append(float *q, const float *k, const float *v, const float *rope, int T, int start,
+                       int nh, int nkv, int hd, float *k_cache, float *v_cache, hipStream_t s,
+                       const PrefillKvF16 *kvf) {
+  PrefillKvF16 f{};
+  if (use_f16_planes(kvf, hd)) {
+    f = *kvf;
+    const int kvw = nkv * hd, P = start + T;
+    if (((P + 15) & ~15) > f.positions || f.kvw != kvw || kvw % 32)
+      return set_error(LLRS_E_INVALID, "prefill attention: f16 K/V scratch of %d positions x %d for %d x %d",
+                       f.positions, f.kvw, P, kvw);
+    if (start > 0)  // the rows of earlier calls and chunks (the planes serve every layer in turn)
+      hipLaunchKernelGGL(kv_split_f16_kernel, dim3((unsigned)((start + 15) / 16), (unsigned)((kvw + 63) / 64)),
+                         dim3(256), 0, s, k_cache, v_cache, kvw, start, f.kh, f.kl, f.vh, f.vl);
+  }
+  const dim3 grid((unsigned)((start + T + 15) / 16 - start / 16), (unsigned)(nh + 2 * nkv));
+#define ROPE(D)                                                                                                  \
+  hipLaunchKernelGGL(rope_append_kernel<D>, grid, dim3(256), 0, s, q, k, v, rope, T, start, nh, nkv, k_cache, \
+                     v_cache, f.kh, f.kl, f.vh, f.vl)
+  switch (hd) {
+    case 16: ROPE(16); break;
+    case 32: ROPE(32); break;
+    case 64: ROPE(64); break;
+    case 128: ROPE(128); break;
+    default: return set_error(LLRS_E_UNSUPPORTED, "attention head_dim %d is not supported", hd);
+  }
+#undef ROPE
+  LLRS_HIP(hipGetLastError());
+  return LLRS_OK;
+}
+
 int launch_attention_rows(const float *q, const float *k_cache, const float *v_cache, int T,
                           int start, int nh, int nkv, int hd, float scale, f16 *out, f16 *out_lo,
-                          hipStream_t s, const PrefillKvF16 *kvf) {
+                          hipStream_t s, const PrefillKvF16 *kvf, f16 *xs, f16 *xs_lo, int ldxs) {
   if (T <= 0 || nkv <= 0 || nh % nkv)
     return set_error(LLRS_E_UNSUPPORTED, "attention over %d rows with %d/%d heads", T, nh, nkv);
   const dim3 grid((unsigned)((T + 15) / 16), (unsigned)nh);
-  if (kvf && hd >= 32 && prefill_attention_f16()) {
-    const int kvw = nkv * hd, P = start + T;
-    if (((P + 15) & ~15) > kvf->positions || kvf->kvw != kvw || kvw % 32)
-      return set_error(LLRS_E_INVALID, "prefill attention: f16 K/V scratch of %d positions x %d for %d x %d",
-                       kvf->positions, kvf->kvw, P, kvw);
-    hipLaunchKernelGGL(kv_split_f16_kernel, dim3((unsigned)((P + 15) / 16), (unsigned)((kvw + 63) / 64)),
-                       dim3(256), 0, s, k_cache, v_cache, kvw, P, kvf->kh, kvf->kl, kvf->vh, kvf->vl);
+  if (use_f16_planes(kvf, hd)) {
 #define ATT16(D)                                                                                      \
   hipLaunchKernelGGL(attention_f16_kernel<D>, grid, dim3(256), 0, s, q, kvf->kh, kvf->kl, kvf->vh, kvf->vl, \
-                     v_cache, T, start, nh, nkv, scale, out, out_lo)
+                     v_cache, T, start, nh, nkv, scale, out, out_lo, xs, xs_lo, ldxs)
     switch (hd) {
       case 32: ATT16(32); break;
       case 64: ATT16(64); break;
@@ -1373,6 +1468,7 @@ int launch_attention_rows(const float *q, const float *k_cache, const float *v_c
   }
 #undef ATT
   LLRS_HIP(hipGetLastError());
+  if (xs) return launch_xsum_f16(out, out_lo, nh * hd, nh * hd, T, xs, xs_lo, ldxs, s);
   return LLRS_OK;
 }
 

@@ -66,3 +66,34 @@ def test_prefill_quantized_weights(llrs, backend, oracle, tmp_path, hidden, head
                            recipe=getattr(llrs.LoadQuantization, recipe))
     model = llrs.HipQwen2Model.synthetic(backend, cfg)
     check(llrs, oracle, model, tmp_path, cfg.vocab_size, cfg.num_hidden_layers, n, 57 + n)
+
+
+@pytest.mark.parametrize("hd", [16, 32, 64, 128])
+def test_prefill_chunks_and_unaligned_start(llrs, backend, oracle, tmp_path, hd):
+    """37 tokens, then 2,063 from position 37: the second call grows the row
+    buffers, starts inside a 16-position block of the f16 K/V planes, and runs
+    as a 2,048-row chunk and a 15-row one (position 2,085 starts inside a block
+    again); in one call of 2,100 the last chunk starts at a block's edge.
+    hidden 1,024 with Q4_K o (its sums come from the attention kernel, or from
+    a pass of their own at head_dim 16)."""
+    cfg = llrs.SynthConfig(hidden_size=1024, intermediate_size=1024, num_attention_heads=1024 // hd,
+                           num_key_value_heads=256 // hd, num_hidden_layers=2, vocab_size=500,
+                           max_position_embeddings=2304, seed=63, tie_word_embeddings=False)
+    model = llrs.HipQwen2Model.synthetic(backend, cfg)
+    model.export_gguf(tmp_path / "m.gguf")
+    om = oracle.load(tmp_path / "m.gguf")
+    om.new_state(2104)
+    prompt = np.random.default_rng(63).integers(0, cfg.vocab_size, 2100).astype(np.uint32)
+    om.prefill(prompt, 0)
+    for cut in (37, 0):
+        kv = llrs.KVCache(model, 2104)
+        if cut:
+            model.prefill(prompt[:cut], 0, kv)
+        model.prefill(prompt[cut:], cut, kv)
+        err = float(np.abs(kv.logits() - om.logits()).max())
+        print(f"[chunks] hd={hd} cut={cut} logits max-abs err {err:.3e}", flush=True)
+        assert err <= 2e-4 * max(1.0, float(np.abs(om.logits()).max()))
+        for layer in range(cfg.num_hidden_layers):
+            for which in ("k", "v"):
+                a, b = kv.layer(layer, which, 2100), om.kv(layer, which, 2100)
+                assert float(np.abs(a - b).max()) <= 2e-5 * max(1.0, float(np.abs(b).max())), (layer, which)
