@@ -106,6 +106,9 @@ struct llrs_backend {
   // Scratch device buffers for the host-pointer matvec entry point.
   float *x_dev = nullptr, *y_dev = nullptr;
   size_t x_cap = 0, y_cap = 0;
+  // Pinned staging of the same entry point, h_cap floats: x, then y.
+  float *h_buf = nullptr;
+  size_t h_cap = 0;
   std::atomic<int> refs{1};  // the creator's handle + one per tensor and model
 };
 

@@ -70,6 +70,10 @@ struct AttnArgs {
 int launch_embed(const llrs_tensor *emb, const uint32_t *tok_by_pos, const int *pos, int max_seq,
                  float *out, unsigned *epoch, hipStream_t s, unsigned *clear = nullptr,
                  int nclear = 0);
+// dst[0 .. n) = src[0 .. n), or `one` for n = 1 without src; *pos = pos_value if
+// pos is set.  Either side may be pinned host memory.
+int launch_copy_words(uint32_t *dst, const uint32_t *src, uint32_t one, size_t n, int *pos, int pos_value,
+                      hipStream_t s);
 int launch_rmsnorm(const float *in, const float *w, float *out, int n, float eps, hipStream_t s);
 long attention_part_stride(int hd);
 size_t attention_scratch_words(int nh, int hd, int max_seq);

@@ -154,6 +154,19 @@ __global__ void advance_kernel(int *pos, int max_seq) {
   *pos = p > max_seq ? max_seq : p;
 }
 
+// A call's input or output between pinned host memory and the device, with the
+// position it is for.  A kernel in the stream's own queue: a copy of the runtime
+// costs host time and a wait between queues (staging a decode step's token and
+// position by two of them, and reading the wait flags by two more, made a step
+// 32 us longer).
+__global__ __launch_bounds__(256) void copy_words_kernel(uint32_t *__restrict__ dst,
+                                                         const uint32_t *__restrict__ src, uint32_t one, size_t n,
+                                                         int *pos, int pos_value) {
+  const size_t step = (size_t)gridDim.x * 256, i0 = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i0 == 0 && pos) *pos = pos_value;
+  for (size_t i = i0; i < n; i += step) dst[i] = src ? src[i] : one;
+}
+
 // Plain streaming copy (the calibration copy of llrs_device_copy).
 __global__ __launch_bounds__(256) void copy_kernel(uint4 *__restrict__ dst,
                                                    const uint4 *__restrict__ src, size_t n16) {
@@ -170,6 +183,15 @@ int launch_embed(const llrs_tensor *emb, const uint32_t *tok_by_pos, const int *
   hipLaunchKernelGGL(embed_kernel, dim3((n + 255) / 256), dim3(256), 0, s, emb->dev, emb->type,
                      emb->row_bytes, H, (uint32_t)emb->rows, tok_by_pos, pos, max_seq, out, epoch,
                      clear, nclear);
+  LLRS_HIP(hipGetLastError());
+  return LLRS_OK;
+}
+
+int launch_copy_words(uint32_t *dst, const uint32_t *src, uint32_t one, size_t n, int *pos, int pos_value,
+                      hipStream_t s) {
+  if (n > 1 && !src) return set_error(LLRS_E_INVALID, "copy of %zu words without a source", n);
+  const size_t blocks = std::max<size_t>(1, std::min<size_t>(1024, (n + 255) / 256));
+  hipLaunchKernelGGL(copy_words_kernel, dim3((unsigned)blocks), dim3(256), 0, s, dst, src, one, n, pos, pos_value);
   LLRS_HIP(hipGetLastError());
   return LLRS_OK;
 }

@@ -119,7 +119,7 @@ __device__ void bar_wait(unsigned *bar, unsigned *err, int nwg, unsigned k, bool
         if (!t0) {
           t0 = t;
         } else if (t - t0 > 2000000ull) {  // 20 ms
-          if (lane == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (lane == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
           break;
         }
       }

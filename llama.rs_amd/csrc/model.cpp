@@ -81,7 +81,11 @@ struct llrs_kv {
         *rope = nullptr;
   unsigned long long *scores = nullptr;  // attention chunk partials, tagged words
   unsigned *epoch = nullptr;             // the step's tag, advanced by the embedding
-  unsigned *attn_err = nullptr;          // an attention merge gave up waiting
+  // A wait gave up: [0] a persistent-decode barrier, [1] an attention merge.  In
+  // pinned memory: kernels only ever set them, and every synchronous call reads
+  // them, which from device memory took two blocking copies.
+  unsigned *wait_flags = nullptr, *flags_dev = nullptr;  // host and device address
+  unsigned *attn_err = nullptr;                          // flags_dev + 1
   llrs::SampleScratch sample;            // llrs_sample's buffers, allocated on first use
   int *pos = nullptr;
   uint32_t *tok_by_pos = nullptr, *next_token = nullptr;
@@ -1008,11 +1012,10 @@ static int setup_persistent(llrs_model *m, llrs_kv *kv) {
   } else {
     LLRS_TRY(A((void **)&kv->p_bar, kPersistentBarWords * 4));
   }
-  LLRS_TRY(A((void **)&kv->p_err, 64));
+  kv->p_err = kv->flags_dev;
   hipStream_t s = m->b->stream;
   LLRS_HIP(hipMemcpyAsync(kv->p_layers, host.data(), nl * sizeof(PersistentLayer), hipMemcpyHostToDevice, s));
   LLRS_HIP(hipMemsetAsync(kv->p_bar, 0, kPersistentBarWords * 4, s));
-  LLRS_HIP(hipMemsetAsync(kv->p_err, 0, 64, s));
   LLRS_HIP(hipStreamSynchronize(s));
   memcpy(kv->p_types, t, sizeof t);
   kv->p_act_stride = (long)(per_layer / 4);
@@ -1023,10 +1026,8 @@ static int setup_persistent(llrs_model *m, llrs_kv *kv) {
 
 // Clears the device-side wait flags (outside any graph capture).
 static int clear_wait_flags(llrs_kv *kv) {
-  hipStream_t s = kv->m->b->stream;
-  if (kv->p_err) LLRS_HIP(hipMemsetAsync(kv->p_err, 0, 4, s));
-  LLRS_HIP(hipMemsetAsync(kv->attn_err, 0, 4, s));
-  LLRS_HIP(hipStreamSynchronize(s));
+  LLRS_HIP(hipStreamSynchronize(kv->m->b->stream));
+  kv->wait_flags[0] = kv->wait_flags[1] = 0;
   return LLRS_OK;
 }
 
@@ -1035,9 +1036,8 @@ static int clear_wait_flags(llrs_kv *kv) {
 // reported: the steps since the last check are untrustworthy (their K/V rows
 // too, so the cache should be prefilled again), but later calls run normally.
 static int check_persistent(llrs_kv *kv) {
-  unsigned err = 0, aerr = 0;
-  if (kv->p_err) LLRS_HIP(hipMemcpy(&err, kv->p_err, 4, hipMemcpyDeviceToHost));
-  LLRS_HIP(hipMemcpy(&aerr, kv->attn_err, 4, hipMemcpyDeviceToHost));
+  const volatile unsigned *f = kv->wait_flags;
+  const unsigned err = f[0], aerr = f[1];
   if (!err && !aerr) return LLRS_OK;
   LLRS_TRY(clear_wait_flags(kv));
   if (err) return set_error(LLRS_E_HIP, "persistent decode: a device-wide barrier timed out");
@@ -1058,6 +1058,7 @@ static void free_kv(llrs_kv *kv) {
   for (void *p : kv->pf_allocs) (void)hipFree(p);
   if (kv->p_bar_uc) uc_release(kv->p_bar);
   if (kv->pinned) (void)hipHostFree(kv->pinned);
+  if (kv->wait_flags) (void)hipHostFree(kv->wait_flags);
   delete kv;
   free_model(m);
 }
@@ -1085,7 +1086,7 @@ static int kv_create_impl(llrs_model *m, size_t max_seq, llrs_kv **out) {
       (rc = A((void **)&kv->act, F * 4)) || (rc = A((void **)&kv->logits, c.vocab_size * 4)) ||
       (rc = A((void **)&kv->scores, attention_scratch_words((int)c.num_attention_heads,
                                                             (int)c.head_dim, (int)max_seq) * 8)) ||
-      (rc = A((void **)&kv->epoch, 64)) || (rc = A((void **)&kv->attn_err, 64)) ||
+      (rc = A((void **)&kv->epoch, 64)) ||
       (rc = A((void **)&kv->rope, max_seq * c.head_dim * 4)) || (rc = A((void **)&kv->pos, 64)) ||
       (rc = A((void **)&kv->tok_by_pos, (max_seq + 1) * 4)) || (rc = A((void **)&kv->next_token, 64)) ||
       (rc = A((void **)&kv->amax_key, 64)) || (rc = A((void **)&kv->done, 64)) ||
@@ -1099,6 +1100,15 @@ static int kv_create_impl(llrs_model *m, size_t max_seq, llrs_kv **out) {
     free_kv(kv);
     return set_error(LLRS_E_OOM, "hipHostMalloc failed: %s", hipGetErrorString(e));
   }
+  e = hipHostMalloc((void **)&kv->wait_flags, 64, hipHostMallocMapped | hipHostMallocCoherent);
+  if (e != hipSuccess) kv->wait_flags = nullptr;
+  if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&kv->flags_dev, kv->wait_flags, 0);
+  if (e != hipSuccess) {
+    free_kv(kv);
+    return set_error(LLRS_E_OOM, "hipHostMalloc failed: %s", hipGetErrorString(e));
+  }
+  kv->wait_flags[0] = kv->wait_flags[1] = 0;
+  kv->attn_err = kv->flags_dev + 1;
   std::vector<float> rope(max_seq * c.head_dim);
   rope_table(rope.data(), max_seq, c.head_dim, c.rope_theta);
   hipStream_t s = m->b->stream;
@@ -1118,7 +1128,6 @@ static int kv_create_impl(llrs_model *m, size_t max_seq, llrs_kv **out) {
     e = hipMemsetAsync(kv->scores, 0,
                        attention_scratch_words((int)c.num_attention_heads, (int)c.head_dim, (int)max_seq) * 8, s);
   if (e == hipSuccess) e = hipMemsetAsync(kv->epoch, 0, 64, s);
-  if (e == hipSuccess) e = hipMemsetAsync(kv->attn_err, 0, 64, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
     free_kv(kv);
@@ -1135,12 +1144,13 @@ static int kv_create_impl(llrs_model *m, size_t max_seq, llrs_kv **out) {
 // Stages tok_by_pos[pos .. pos+n) = tokens and *pos = pos on the device.
 static int stage_tokens(llrs_kv *kv, const uint32_t *tokens, size_t n, size_t pos) {
   hipStream_t s = kv->m->b->stream;
-  LLRS_HIP(hipStreamSynchronize(s));  // the pinned staging buffer is free again
-  memcpy(kv->pinned, tokens, n * 4);
-  kv->pinned[n] = (uint32_t)pos;
-  if (n) LLRS_HIP(hipMemcpyAsync(kv->tok_by_pos + pos, kv->pinned, n * 4, hipMemcpyHostToDevice, s));
-  LLRS_HIP(hipMemcpyAsync(kv->pos, kv->pinned + n, 4, hipMemcpyHostToDevice, s));
-  return LLRS_OK;
+  const uint32_t *src = nullptr;
+  if (n > 1) {
+    LLRS_HIP(hipStreamSynchronize(s));  // the pinned staging buffer is free again
+    memcpy(kv->pinned, tokens, n * 4);
+    LLRS_HIP(hipHostGetDevicePointer((void **)&src, kv->pinned, 0));
+  }
+  return launch_copy_words(kv->tok_by_pos + pos, src, n ? tokens[0] : 0, n, kv->pos, (int)pos, s);
 }
 
 // Rows of one prefill chunk: bounds the prefill buffers (7B: 0.54 GB).  Longer
@@ -1386,9 +1396,9 @@ static int prefill_batched(llrs_model *m, llrs_kv *kv, size_t start, size_t n) {
     }
     last_rows = (size_t)T;
   }
-  LLRS_HIP(hipMemcpyAsync(kv->residual, kv->pf_x + (last_rows - 1) * H, (size_t)H * 4,
-                          hipMemcpyDeviceToDevice, s));
-  LLRS_TRY(launch_set_pos(kv->pos, (int)(start + n - 1), s));
+  LLRS_TRY(launch_copy_words(reinterpret_cast<uint32_t *>(kv->residual),
+                             reinterpret_cast<const uint32_t *>(kv->pf_x + (last_rows - 1) * H), 0, (size_t)H,
+                             kv->pos, (int)(start + n - 1), s));
   return launch_projection(m, kv, 0, P_LM_HEAD, s);
 }
 
@@ -1626,8 +1636,8 @@ int llrs_kv_debug_set_wait_flag(llrs_kv *kv, int which) {
   if (which != 0 && which != 1) return set_error(LLRS_E_INVALID, "unknown wait flag %d", which);
   if (which == 0 && !kv->p_err) return set_error(LLRS_E_INVALID, "the cache has no persistent decode");
   LLRS_HIP(hipSetDevice(kv->m->b->device));
-  const unsigned one = 1;
-  LLRS_HIP(hipMemcpy(which == 0 ? kv->p_err : kv->attn_err, &one, 4, hipMemcpyHostToDevice));
+  LLRS_HIP(hipStreamSynchronize(kv->m->b->stream));
+  kv->wait_flags[which] = 1;
   return LLRS_OK;
 }
 

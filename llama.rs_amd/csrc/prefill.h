@@ -115,6 +115,5 @@ int launch_attention_rows(const float *q, const float *k_cache, const float *v_c
 // with xs set, also their 32-column sums per row.
 int launch_swiglu_f16(const float *g, const float *u, f16 *out, f16 *out_lo, size_t n, int cols, hipStream_t s,
                       f16 *xs = nullptr, f16 *xs_lo = nullptr, int ldxs = 0);
-int launch_set_pos(int *pos, int value, hipStream_t s);
 
 }  // namespace llrs

@@ -1041,7 +1041,6 @@ __global__ __launch_bounds__(256) void swiglu_f16_kernel(const float *__restrict
   }
 }
 
-__global__ void set_pos_kernel(int *pos, int value) { *pos = value; }
 
 
 // C[t][j] = (C[t][j] when accumulating, else bias[j] or 0) + the split-K
@@ -1482,10 +1481,5 @@ int launch_swiglu_f16(const float *g, const float *u, f16 *out, f16 *out_lo, siz
   return LLRS_OK;
 }
 
-int launch_set_pos(int *pos, int value, hipStream_t s) {
-  hipLaunchKernelGGL(set_pos_kernel, dim3(1), dim3(1), 0, s, pos, value);
-  LLRS_HIP(hipGetLastError());
-  return LLRS_OK;
-}
 
 }  // namespace llrs

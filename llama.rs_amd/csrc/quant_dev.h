@@ -182,7 +182,7 @@ __device__ __forceinline__ bool tagged_wait_over(unsigned long long &t0, unsigne
   const unsigned long long t = wall_clock64();
   if (!t0) t0 = t;
   if (t - t0 < 2000000ull) return false;
-  if (err && (thread_x() & 63) == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (err && (thread_x() & 63) == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   return true;
 }
 
