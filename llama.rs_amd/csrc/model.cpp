@@ -723,6 +723,29 @@ static FastGemvArgs projection_args(llrs_model *m, llrs_kv *kv, size_t l, int wh
 
 // The decode step's launch(es) for projection group `which` of layer `l`; the
 // bench's per-kernel timing calls this same function.
+// The unquantized products of `ws` (one type and row length) behind one norm.
+static bool float_group(std::initializer_list<const llrs_tensor *> ws) {
+  const llrs_tensor *a = *ws.begin();
+  for (const llrs_tensor *w : ws)
+    if (!gemv_float_norm_supports(w) || w->type != a->type || w->cols != a->cols) return false;
+  return true;
+}
+
+static GemvFloatArgs float_args(llrs_kv *kv, const float *norm, const llrs_tensor *w, float *out,
+                                const float *bias = nullptr) {
+  GemvFloatArgs a{};
+  a.w[0] = w->dev;
+  a.rows[0] = (int)w->rows;
+  a.out[0] = out;
+  a.bias[0] = bias;
+  a.row_bytes = w->row_bytes;
+  a.cols = (int)w->cols;
+  a.x = kv->residual;
+  a.norm = norm;
+  a.eps = kv->m->cfg.rms_norm_eps;
+  return a;
+}
+
 static int launch_projection(llrs_model *m, llrs_kv *kv, size_t l, int which, hipStream_t s) {
   const llrs_model_config &c = m->cfg;
   const int H = (int)c.hidden_size, F = (int)c.intermediate_size;
@@ -739,20 +762,35 @@ static int launch_projection(llrs_model *m, llrs_kv *kv, size_t l, int which, hi
     return launch_gemv_fast(a, fast_grid(m, a, which == P_GATE_UP), s);
   }
   if (which == P_LM_HEAD) {
-    LLRS_TRY(launch_rmsnorm(kv->residual, m->norm, kv->hidden, H, eps, s));
-    LLRS_TRY(launch_gemv_generic(m->lm_head, kv->hidden, kv->logits, nullptr, false, s));
+    if (float_group({m->lm_head})) {
+      LLRS_TRY(launch_gemv_float_norm(float_args(kv, m->norm, m->lm_head, kv->logits), m->lm_head->type, false, m->b->cu_count, s));
+    } else {
+      LLRS_TRY(launch_rmsnorm(kv->residual, m->norm, kv->hidden, H, eps, s));
+      LLRS_TRY(launch_gemv_generic(m->lm_head, kv->hidden, kv->logits, nullptr, false, s));
+    }
     return launch_argmax(kv->logits, (int)c.vocab_size, kv->pos, (int)kv->max_seq_len,
                          kv->tok_by_pos, kv->next_token, 1, s);
   }
   DevLayer &L = m->layers[l];
   switch (which) {
     case P_QKV:
+      if (float_group({L.q, L.k, L.v})) {
+        GemvFloatArgs a = float_args(kv, L.attn_norm, L.q, kv->q, L.bq);
+        a.w[1] = L.k->dev, a.rows[1] = (int)L.k->rows, a.out[1] = kv->k, a.bias[1] = L.bk;
+        a.w[2] = L.v->dev, a.rows[2] = (int)L.v->rows, a.out[2] = kv->v, a.bias[2] = L.bv;
+        return launch_gemv_float_norm(a, L.q->type, false, m->b->cu_count, s);
+      }
       LLRS_TRY(launch_rmsnorm(kv->residual, L.attn_norm, kv->hidden, H, eps, s));
       LLRS_TRY(launch_gemv_generic(L.q, kv->hidden, kv->q, L.bq, false, s));
       LLRS_TRY(launch_gemv_generic(L.k, kv->hidden, kv->k, L.bk, false, s));
       return launch_gemv_generic(L.v, kv->hidden, kv->v, L.bv, false, s);
     case P_O: return launch_gemv_generic(L.o, kv->attn, kv->residual, nullptr, true, s);
     case P_GATE_UP:
+      if (float_group({L.gate, L.up})) {
+        GemvFloatArgs a = float_args(kv, L.ffn_norm, L.gate, kv->act);
+        a.w[1] = L.up->dev, a.rows[1] = (int)L.up->rows;
+        return launch_gemv_float_norm(a, L.gate->type, true, m->b->cu_count, s);
+      }
       LLRS_TRY(launch_rmsnorm(kv->residual, L.ffn_norm, kv->hidden, H, eps, s));
       LLRS_TRY(launch_gemv_generic(L.gate, kv->hidden, kv->gate, nullptr, false, s));
       LLRS_TRY(launch_gemv_generic(L.up, kv->hidden, kv->up, nullptr, false, s));
