@@ -1274,15 +1274,15 @@ static PrefillGemmArgs rows_of(const PrefillGemmArgs &g, int from, int rows) {
 static bool takes_big(const PrefillGemmArgs &g) {
   if (g.t <= 64 || g.type == LLRS_F16 || g.type == LLRS_BF16) return false;
   const int tile = prefill_reg_big_row_tile(g.type, g.w2 != nullptr), rows = g.w2 ? g.dual_rows : g.n;
-  const long tiles = (long)((rows + tile - 1) / tile) * ((g.t + 63) / 64), slots = gemm_slots();
+  const long tiles = (long)((rows + tile - 1) / tile) * ((g.t + 63) / 64), slots = gemm_slots() / 2;
   return 2 * tiles <= slots || 4 * tiles >= 3 * slots;
 }
 
-// Register-decoded products over many tokens, two workgroups a CU: whole rounds
+// Register-decoded products over many tokens, one workgroup a CU: whole rounds
 // of tiles run as they are; a last round that would fill at most half the
 // slots (or a product with fewer tiles than slots) splits K over them.
 static int launch_reg_big(const PrefillGemmArgs &g, hipStream_t s) {
-  const int slots = gemm_slots(), nb = (g.k + 255) / 256;
+  const int slots = gemm_slots() / 2, nb = (g.k + 255) / 256;
   const int tile = prefill_reg_big_row_tile(g.type, g.w2 != nullptr), rows = g.w2 ? g.dual_rows : g.n;
   const int nt = (rows + tile - 1) / tile, mt = (g.t + 63) / 64;
   auto splits = [&](int tiles, int n) {

@@ -286,6 +286,44 @@ __device__ __forceinline__ void multiply(f32x4 (&acc)[TT][RT], B &blk, const Row
   }
 }
 
+// Step s of a buffer with its operands wh decoded, while those of the step after it
+// are decoded (ahead) in the MFMAs' shadow: two VALU operations after each, the
+// fragments one token tile early.
+template <uint32_t TY, int TT, int RT, int SA>
+__device__ __forceinline__ void multiply_ahead(f32x4 (&acc)[TT][RT], const Row<TY> (&w)[RT], half8 (&wh)[RT],
+                                               const uint8_t *frag, int step, bool ahead, int kg) {
+  half8 nh[RT], none;
+  if (ahead) {
+#pragma unroll
+    for (int r = 0; r < RT; r++) w[r].weight(step + 1, kg, nh[r], none);
+  }
+  const int s = step % SA;
+#pragma unroll
+  for (int i = 0; i < TT; i++) {
+    const half8 ah = *reinterpret_cast<const half8 *>(frag + (s * TT + i) * 1024);
+    const half8 al = *reinterpret_cast<const half8 *>(frag + ((SA + s) * TT + i) * 1024);
+#pragma unroll
+    for (int r = 0; r < RT; r++) acc[i][r] = mfma(al, wh[r], acc[i][r]);
+#pragma unroll
+    for (int r = 0; r < RT; r++) acc[i][r] = mfma(ah, wh[r], acc[i][r]);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x100, 2 + RT, 0);  // LDS reads
+#pragma unroll
+  for (int i = 0; i < TT; i++) {
+    if (i + 1 < TT) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+    for (int m = 0; m < 2 * RT; m++) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // an MFMA
+      __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);  // VALU
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (ahead) {
+#pragma unroll
+    for (int r = 0; r < RT; r++) wh[r] = nh[r];
+  }
+}
+
 // A block type's unit in absolute terms: d times its sums (a block with d = 0
 // has finite sums and adds its dmin term only), and for Q4_K - dmin * sum_s m_s
 // xsum_s over the block's eight sub-blocks: lane group kg contributes
@@ -633,20 +671,23 @@ __global__ __launch_bounds__(64 * (kMaxRowWaves + 1) * KW, 3) void prefill_reg_k
                               kq == 0 && wave < nrw);
 }
 
-// The same products over many tokens: 64 tokens x four waves of 16 RT rows, two
-// workgroups a CU, whole K ranges; the row waves stage the activations
-// themselves (their loads go out before the next unit's rows, and each has a
-// buffer's products to land).  The matrix cores bound it: RT = 4 reads 8
-// fragments of LDS per 32 MFMAs, half of LDS's rate at the full MFMA rate
-// (measured: matrix cores 43% busy at the ~1.9 GHz the card then holds).  7B
-// shape, 512 tokens, per layer: gate/up 361 -> 340 us, ffn_down 295 -> 280, q, k
-// and o 100 -> 92 against the LDS-staged kernel with decoded weights in LDS.
+// The same products over many tokens: 64 tokens x eight waves of 16 RT rows, one
+// workgroup a CU, whole K ranges; the row waves stage the activations themselves
+// (their loads go out before the next unit's rows, and each has a buffer's
+// products to land).  RT = 4 reads 8 fragments of LDS per 32 MFMAs, half of LDS's
+// rate at the full MFMA rate.  What bounds it is spread out: matrix cores busy
+// 45% at the ~1.9 GHz the card then holds, and a half of the MFMAs, all memory
+// latency or half of the decoding taken out win 8% each.  7B shape, 512 tokens, per
+// layer: gate/up 332 us, ffn_down 251; two workgroups of four waves a CU, which
+// load the activations twice and meet twice as often, 340 and 280 (with Q6_K's
+// decoding ahead of the products, as Q4_K's, 300); the LDS-staged kernel with
+// decoded weights in LDS 361 and 295.
 // Four row tiles leave registers for one set of accumulators only, so Q4_K's are
 // kept in units of the row's current d, rescaled by d_prev / d at each block (a
 // block with d = 0 keeps the unit and multiplies zeros), and its dmin * m term
 // is a second, 1/32 as long product at the end: - (dmin m)_s (hi + lo) with
 // xsum_s (hi + lo).
-constexpr int kBigTT = 4, kBigWaves = 4, kBigSA = 2;
+constexpr int kBigTT = 4, kBigWaves = 8, kBigSA = 4;
 constexpr size_t big_acts_bytes() { return (size_t)2 * 2 * kBigSA * kBigTT * 1024; }
 template <uint32_t TY, int RT> constexpr size_t big_lds_bytes() {
   return big_acts_bytes() + kBigWaves * wave_bytes<TY, RT>();
@@ -657,7 +698,7 @@ __global__ __launch_bounds__(64 * kBigWaves, 2) void prefill_reg_big_kernel(Pref
   constexpr bool kRatio = TY == LLRS_Q4_K, kUnits = R::kUnit == kBlock && !kRatio;
   constexpr int TT = kBigTT, SA = kBigSA, NB = R::kCols / (32 * SA), NF = 2 * SA * TT, NL = NF / kBigWaves;
   constexpr int GT = DUAL ? RT / 2 : RT;
-  static_assert(kBigWaves == TT, "wave w stages token tile w");
+  static_assert(kBigWaves == 2 * TT, "waves w and w + TT stage token tile w, half of the steps each");
   extern __shared__ __align__(16) uint8_t lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, kg = lane >> 4;
   const int t0 = blockIdx.y * 16 * TT, T = g.t, K = g.k;
@@ -673,21 +714,23 @@ __global__ __launch_bounds__(64 * kBigWaves, 2) void prefill_reg_big_kernel(Pref
   // This wave's fragments: token tile `wave`, every step, both planes (lane =
   // (token, piece), slots as in prefill_reg_kernel).
   const int at = lane >> 2, ap = lane & 3, slot = 16 * (16 * ap + (at ^ (4 * ap)));
-  const uint32_t arow = (uint32_t)min(t0 + 16 * wave + at, T - 1) * (uint32_t)g.lda + 8 * ap;
+  const int tile = wave % TT, half = wave / TT * (SA / 2);
+  const uint32_t arow = (uint32_t)min(t0 + 16 * tile + at, T - 1) * (uint32_t)g.lda + 8 * ap;
   const f16 *const ahi = g.a, *const alo = g.a_lo;
   half8 st[NL];
   auto load_acts = [&](int k0) INLINE {
 #pragma unroll
     for (int j = 0; j < NL; j++)
-      st[j] = *reinterpret_cast<const half8 *>((j < SA ? ahi : alo) + min(k0 + 32 * (j % SA), ke - 32) + arow);
+      st[j] = *reinterpret_cast<const half8 *>((j < SA / 2 ? ahi : alo) + min(k0 + 32 * (half + j % (SA / 2)), ke - 32) + arow);
   };
   auto store_acts = [&](int k0, int b) INLINE {
 #pragma unroll
     for (int j = 0; j < NL; j++) {
-      uint32_t in = k0 + 32 * (j % SA) < ke ? ~0u : 0u;
+      const int f = j / (SA / 2) * SA + half + j % (SA / 2);
+      uint32_t in = k0 + 32 * (f % SA) < ke ? ~0u : 0u;
       u32x4 v = __builtin_bit_cast(u32x4, st[j]);
       if constexpr (R::kUnit != kBlock) v &= u32x4{in, in, in, in};
-      *reinterpret_cast<u32x4 *>(lds + (b * NF + j * TT + wave) * 1024 + slot) = v;
+      *reinterpret_cast<u32x4 *>(lds + (b * NF + f * TT + tile) * 1024 + slot) = v;
     }
   };
   f32x4 acc[TT][RT], blk[kUnits ? TT : 1][kUnits ? RT : 1];
@@ -723,6 +766,11 @@ __global__ __launch_bounds__(64 * kBigWaves, 2) void prefill_reg_big_kernel(Pref
 #pragma unroll
         for (int r = 0; r < RT; r++) blk[i][r] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    half8 wh[RT], none;
+    if constexpr (kRatio) {
+#pragma unroll
+      for (int r = 0; r < RT; r++) w[r].weight(0, kg, wh[r], none);
+    }
 #pragma unroll
     for (int b = 0; b < NB; b++) {
       const int kn = k0 + 32 * SA * (b + 1);  // the next buffer's columns
@@ -730,10 +778,14 @@ __global__ __launch_bounds__(64 * kBigWaves, 2) void prefill_reg_big_kernel(Pref
       if (next) load_acts(kn);
       if (kMore && b == 0) src.load(k0 + R::kCols);
       __builtin_amdgcn_sched_barrier(0);  // the scheduler would sink the loads to their uses
-      if constexpr (kRatio)
-        multiply<TY, TT, RT, SA>(acc, acc, w, frag0 + (b & 1) * NF * 1024, b, k0, ke, kg);
-      else
-        multiply<TY, TT, RT, SA>(acc, blk, w, frag0 + (b & 1) * NF * 1024, b, k0, ke, kg);
+      const uint8_t *const frag = frag0 + (b & 1) * NF * 1024;
+      if constexpr (kRatio) {
+#pragma unroll
+        for (int step = b * SA; step < (b + 1) * SA; step++)
+          multiply_ahead<TY, TT, RT, SA>(acc, w, wh, frag, step, step + 1 < R::kCols / 32, kg);
+      } else {
+        multiply<TY, TT, RT, SA>(acc, blk, w, frag, b, k0, ke, kg);
+      }
       if constexpr (kUnits)
         if (b + 1 == NB) finish<TY, TT, RT>(acc, blk, w, nullptr, n, kg);
       if (next) store_acts(kn, (b + 1) & 1);
