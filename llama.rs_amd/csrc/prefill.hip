@@ -844,8 +844,10 @@ __global__ __launch_bounds__(256) void rope_append_kernel(float *__restrict__ q,
 // from vth/vtl, 16 output dims a tile).  One score step covers 32 dims where
 // the f32 kernel's covers 4, which moves the kernel off the matrix cores'
 // f32 rate.  HD >= 32.
-template <int HD>
-__global__ __launch_bounds__(256, 3) void attention_f16_kernel(const float *__restrict__ q,
+// QT tiles of 16 query rows a workgroup share the K and V loads, which bound the
+// kernel (16 KB from L2 per tile and 16 keys: 13 TB/s with one tile).
+template <int HD, int QT>
+__global__ __launch_bounds__(256, QT == 1 ? 3 : 2) void attention_f16_kernel(const float *__restrict__ q,
                                                             const f16 *__restrict__ kh,
                                                             const f16 *__restrict__ kl,
                                                             const f16 *__restrict__ vh,
@@ -858,14 +860,17 @@ __global__ __launch_bounds__(256, 3) void attention_f16_kernel(const float *__re
   constexpr int NT = HD / 16;  // 16-dim output tiles
   __shared__ float so[4][16][HD + 4];
   __shared__ float sm[4][16], sl[4][16];
-  const int q0 = (gridDim.x - 1 - blockIdx.x) * 16;  // the longest tiles start first
+  const int q0 = (gridDim.x - 1 - blockIdx.x) * 16 * QT;  // the longest tiles start first
   const int h = blockIdx.y, kvh = h / (nh / nkv), kvw = nkv * HD;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-  const int pmax = start + min(q0 + 15, T - 1);
-  const int pq = start + min(q0 + i, T - 1);  // rows past T mask as the last row
-  half8 qh[NC], ql[NC];
-  {
-    const float *qp = q + (size_t)min(q0 + i, T - 1) * nh * HD + h * HD + 8 * g;
+  const int pmax = start + min(q0 + 16 * QT - 1, T - 1);
+  int pq[QT];  // rows past T mask as the last row
+  half8 qh[QT][NC], ql[QT][NC];
+#pragma unroll
+  for (int u = 0; u < QT; u++) {
+    const int row = min(q0 + 16 * u + i, T - 1);
+    pq[u] = start + row;
+    const float *qp = q + (size_t)row * nh * HD + h * HD + 8 * g;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
       const float4 a = *reinterpret_cast<const float4 *>(qp + 32 * c);
@@ -875,8 +880,8 @@ __global__ __launch_bounds__(256, 3) void attention_f16_kernel(const float *__re
       for (int e = 0; e < 8; e++) {
         f16 hi, lo;
         split_f16(x[e], hi, lo);
-        qh[c][e] = hi;
-        ql[c][e] = lo;
+        qh[u][c][e] = hi;
+        ql[u][c][e] = lo;
       }
     }
   }
@@ -884,10 +889,15 @@ __global__ __launch_bounds__(256, 3) void attention_f16_kernel(const float *__re
   // keys 16 b + 4 g ... (kv_split_f16_kernel's block layout; 16 * kvw halves a block).
   const size_t ko = (size_t)kvh * (HD / 32) * 512 + i * 32 + 8 * g;
   const size_t vo = (size_t)(kvh * HD + i) * 16 + 4 * g;
-  f32x4 o[NT];
+  f32x4 o[QT][NT];
+  float M[QT], L[QT];
 #pragma unroll
-  for (int t = 0; t < NT; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float M = -INFINITY, L = 0.f;
+  for (int u = 0; u < QT; u++) {
+    M[u] = -INFINITY;
+    L[u] = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; t++) o[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   const int nb = pmax / 16 + 1;
   half8 kah[NC], kal[NC];
   half4v vah[NT], val[NT];
@@ -913,106 +923,117 @@ __global__ __launch_bounds__(256, 3) void attention_f16_kernel(const float *__re
   }
   for (int b = wave; b < nb; b += 4) {
     const int key0 = b * 16;
-    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+    f32x4 st[QT];
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-      s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kal[c], qh[c], s0, 0, 0, 0);
-      s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kah[c], ql[c], s1, 0, 0, 0);
-      s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kah[c], qh[c], s0, 0, 0, 0);
+    for (int u = 0; u < QT; u++) {
+      f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kal[c], qh[u][c], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kah[c], ql[u][c], s1, 0, 0, 0);
+        s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kah[c], qh[u][c], s0, 0, 0, 0);
+      }
+      st[u] = s0 + s1;
     }
-    const f32x4 st = s0 + s1;
     if (b + 4 < nb) load_k(key0 + 64);
-    float sc[4], mc = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      sc[r] = key0 + 4 * g + r <= pq ? st[r] * scale : -INFINITY;
-      mc = fmaxf(mc, sc[r]);
-    }
-    mc = fmaxf(mc, lane_partner(mc, 16));
-    mc = fmaxf(mc, lane_partner(mc, 32));
-    const float Mn = fmaxf(M, mc);
-    const bool live = Mn != -INFINITY;
-    const float alpha = live ? expf(M - Mn) : 1.f;
-    float ls = 0.f;
-    half4v ph, pl;
+    for (int u = 0; u < QT; u++) {
+      float sc[4], mc = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const float pw = live ? expf(sc[r] - Mn) : 0.f;
-      ls += pw;
-      f16 hi, lo;
-      split_f16(pw, hi, lo);
-      ph[r] = hi;
-      pl[r] = lo;
-    }
-    L = L * alpha + ls;
-    M = Mn;
+      for (int r = 0; r < 4; r++) {
+        sc[r] = key0 + 4 * g + r <= pq[u] ? st[u][r] * scale : -INFINITY;
+        mc = fmaxf(mc, sc[r]);
+      }
+      mc = fmaxf(mc, lane_partner(mc, 16));
+      mc = fmaxf(mc, lane_partner(mc, 32));
+      const float Mn = fmaxf(M[u], mc);
+      const bool live = Mn != -INFINITY;
+      const float alpha = live ? expf(M[u] - Mn) : 1.f;
+      float ls = 0.f;
+      half4v ph, pl;
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-      o[t] *= alpha;
-      o[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(val[t], ph, o[t], 0, 0, 0);
-      o[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(vah[t], pl, o[t], 0, 0, 0);
-      o[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(vah[t], ph, o[t], 0, 0, 0);
+      for (int r = 0; r < 4; r++) {
+        const float pw = live ? expf(sc[r] - Mn) : 0.f;
+        ls += pw;
+        f16 hi, lo;
+        split_f16(pw, hi, lo);
+        ph[r] = hi;
+        pl[r] = lo;
+      }
+      L[u] = L[u] * alpha + ls;
+      M[u] = Mn;
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        o[u][t] *= alpha;
+        o[u][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(val[t], ph, o[u][t], 0, 0, 0);
+        o[u][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(vah[t], pl, o[u][t], 0, 0, 0);
+        o[u][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(vah[t], ph, o[u][t], 0, 0, 0);
+      }
     }
     if (b + 4 < nb) load_v(key0 + 64);
   }
-  L += lane_partner(L, 16);
-  L += lane_partner(L, 32);
-  if (g == 0) {
-    sm[wave][i] = M;
-    sl[wave][i] = L;
-  }
-  // D layout of O^T: lane (i, g) holds query i, dims 16 t + 4 g + r.
 #pragma unroll
-  for (int t = 0; t < NT; t++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) so[wave][i][16 * t + 4 * g + r] = o[t][r];
-  __syncthreads();
-  // Merge: thread -> query qi, dims c*NT ... c*NT + NT - 1.
-  const int qi = threadIdx.x >> 4, c = threadIdx.x & 15;
-  if (q0 + qi >= T) return;
-  float Mt = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < 4; w++) Mt = fmaxf(Mt, sm[w][qi]);
-  float Lt = 0.f, acc[NT];
-#pragma unroll
-  for (int e = 0; e < NT; e++) acc[e] = 0.f;
-#pragma unroll
-  for (int w = 0; w < 4; w++) {
-    const float mw = sm[w][qi];
-    const float f = mw == -INFINITY ? 0.f : expf(mw - Mt);
-    Lt += sl[w][qi] * f;
-#pragma unroll
-    for (int e = 0; e < NT; e++) acc[e] += so[w][qi][c * NT + e] * f;
-  }
-  const int p = start + q0 + qi;
-  const size_t at = (size_t)(q0 + qi) * nh * HD + h * HD + c * NT;
-  float sum = 0.f;
-  auto emit = [&](int e, float v) {
-    f16 hi, lo;
-    split_f16(v, hi, lo);
-    out[at + e] = hi;
-    out_lo[at + e] = lo;
-    sum += (float)hi + (float)lo;
-  };
-  if (isfinite(Lt) && Lt > 0.f) {
-#pragma unroll
-    for (int e = 0; e < NT; e++) emit(e, acc[e] / Lt);
-  } else {
-    const float *vp = v_cache + (size_t)kvh * HD + c * NT;
-    for (int e = 0; e < NT; e++) {
-      float vs = 0.f;
-      for (int j = 0; j <= p; j++) vs += vp[(size_t)j * kvw + e];
-      emit(e, vs / (float)(p + 1));
+  for (int u = 0; u < QT; u++) {
+    if (u) __syncthreads();  // the tile before has been merged
+    L[u] += lane_partner(L[u], 16);
+    L[u] += lane_partner(L[u], 32);
+    if (g == 0) {
+      sm[wave][i] = M[u];
+      sl[wave][i] = L[u];
     }
-  }
-  // The output's 32-column sums, 32 / NT lanes of the query's 16: in a pass of
-  // their own (xsum_f16_kernel) they took 4.4 us for 24 tokens; nothing here.
-  if (xs) {
+    // D layout of O^T: lane (i, g) holds query i, dims 16 t + 4 g + r.
 #pragma unroll
-    for (int b = 1; b < 32 / NT; b <<= 1) sum += lane_partner(sum, b);
-    if (c % (32 / NT) == 0) {
-      const size_t o = (size_t)(q0 + qi) * ldxs + (h * HD + c * NT) / 32;
-      split_f16(sum, xs[o], xs_lo[o]);
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) so[wave][i][16 * t + 4 * g + r] = o[u][t][r];
+    __syncthreads();
+    // Merge: thread -> query qi, dims c*NT ... c*NT + NT - 1.
+    const int qi = threadIdx.x >> 4, c = threadIdx.x & 15;
+    if (q0 + 16 * u + qi >= T) continue;
+    float Mt = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < 4; w++) Mt = fmaxf(Mt, sm[w][qi]);
+    float Lt = 0.f, acc[NT];
+#pragma unroll
+    for (int e = 0; e < NT; e++) acc[e] = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      const float mw = sm[w][qi];
+      const float f = mw == -INFINITY ? 0.f : expf(mw - Mt);
+      Lt += sl[w][qi] * f;
+#pragma unroll
+      for (int e = 0; e < NT; e++) acc[e] += so[w][qi][c * NT + e] * f;
+    }
+    const int p = start + q0 + 16 * u + qi;
+    const size_t at = (size_t)(q0 + 16 * u + qi) * nh * HD + h * HD + c * NT;
+    float sum = 0.f;
+    auto emit = [&](int e, float v) {
+      f16 hi, lo;
+      split_f16(v, hi, lo);
+      out[at + e] = hi;
+      out_lo[at + e] = lo;
+      sum += (float)hi + (float)lo;
+    };
+    if (isfinite(Lt) && Lt > 0.f) {
+#pragma unroll
+      for (int e = 0; e < NT; e++) emit(e, acc[e] / Lt);
+    } else {
+      const float *vp = v_cache + (size_t)kvh * HD + c * NT;
+      for (int e = 0; e < NT; e++) {
+        float vs = 0.f;
+        for (int j = 0; j <= p; j++) vs += vp[(size_t)j * kvw + e];
+        emit(e, vs / (float)(p + 1));
+      }
+    }
+    // The output's 32-column sums, 32 / NT lanes of the query's 16: in a pass of
+    // their own (xsum_f16_kernel) they took 4.4 us for 24 tokens; nothing here.
+    if (xs) {
+#pragma unroll
+      for (int b = 1; b < 32 / NT; b <<= 1) sum += lane_partner(sum, b);
+      if (c % (32 / NT) == 0) {
+        const size_t o = (size_t)(q0 + 16 * u + qi) * ldxs + (h * HD + c * NT) / 32;
+        split_f16(sum, xs[o], xs_lo[o]);
+      }
     }
   }
 }
@@ -1058,7 +1079,7 @@ __global__ void split_reduce_kernel(float *__restrict__ c, int ldc, const float 
 
 // split_reduce_kernel for a dual gate/up product: row f of gate is virtual
 // column (f / 64) * 128 + f % 64, of up that + 64; h + hl [t][f] = silu(g) * u
-// of the partial sums (split order), as swiglu_tile writes it, and with xso
+// of the partial sums (split order), as the dual products write it, and with xso
 // the 32-column sums (half_wave_xsum).
 __global__ __launch_bounds__(256) void split_reduce_swiglu_kernel(const float *__restrict__ part, int nv, int t_rows,
                                                                   int ksplit, int rows, f16 *__restrict__ h,
@@ -1442,9 +1463,18 @@ int launch_attention_rows(const float *q, const float *k_cache, const float *v_c
     return set_error(LLRS_E_UNSUPPORTED, "attention over %d rows with %d/%d heads", T, nh, nkv);
   const dim3 grid((unsigned)((T + 15) / 16), (unsigned)nh);
   if (use_f16_planes(kvf, hd)) {
-#define ATT16(D)                                                                                      \
-  hipLaunchKernelGGL(attention_f16_kernel<D>, grid, dim3(256), 0, s, q, kvf->kh, kvf->kl, kvf->vh, kvf->vl, \
-                     v_cache, T, start, nh, nkv, scale, out, out_lo, xs, xs_lo, ldxs)
+    const dim3 grid2((unsigned)((T + 31) / 32), (unsigned)nh);
+    // Two tiles of query rows a workgroup while every CU still gets one (fewer
+    // would leave CUs idle behind workgroups of twice the length): 2,000 rows of 12
+    // heads 169 us against 231 with one, 512 rows of 28 heads 28 against 39.
+    const bool two = (long)grid2.x * nh >= gemm_slots() / 2;
+#define ATT16(D)                                                                                            \
+  if (two)                                                                                                  \
+    hipLaunchKernelGGL((attention_f16_kernel<D, 2>), grid2, dim3(256), 0, s, q, kvf->kh, kvf->kl, kvf->vh,  \
+                       kvf->vl, v_cache, T, start, nh, nkv, scale, out, out_lo, xs, xs_lo, ldxs);           \
+  else                                                                                                      \
+    hipLaunchKernelGGL((attention_f16_kernel<D, 1>), grid, dim3(256), 0, s, q, kvf->kh, kvf->kl, kvf->vh,   \
+                       kvf->vl, v_cache, T, start, nh, nkv, scale, out, out_lo, xs, xs_lo, ldxs)
     switch (hd) {
       case 32: ATT16(32); break;
       case 64: ATT16(64); break;
