@@ -1289,8 +1289,9 @@ static PrefillGemmArgs rows_of(const PrefillGemmArgs &g, int from, int rows) {
 
 // Whether the many-token kernel takes a register-decoded product: past one
 // 64-token tile, unless its tiles neither fill three quarters of the slots nor
-// leave room to split K (7B gate/up over 128 tokens, 296 tiles of 512 slots:
-// 137 us against 112; over 256: 187 against 214).  Q6_K ffn_down of 7B over 128
+// leave room to split K (measured with workgroups of half the waves: 7B gate/up
+// over 128 tokens, 296 tiles for 512 slots, 137 us against 112; over 256, 187
+// against 214).  Q6_K ffn_down of 7B over 128
 // tokens: 78 us against 96, q and k over 256: 31 against 35, over 128 equal.
 static bool takes_big(const PrefillGemmArgs &g) {
   if (g.t <= 64 || g.type == LLRS_F16 || g.type == LLRS_BF16) return false;
